@@ -390,7 +390,7 @@ HL_API hl_status hl_context_destroy(hl_context* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     while (!c->externals.empty()) (void)release_external(c->externals.back());
-    for (DevBuf* b : {&c->hot, &c->cull, &c->geom, &c->bits, &c->summary, &c->raw, &c->markq, &c->shadeq,
+    for (DevBuf* b : {&c->hot, &c->cull, &c->geom, &c->bits, &c->summary, &c->raw, &c->markq, &c->columns, &c->shadeq,
                       &c->words, &c->accum, &c->vogel, &c->rcirr, &c->tilebin})
         if (b->p) (void)hipFree(b->p);
     delete c;
@@ -630,11 +630,16 @@ HL_API hl_status hl_light_cull_clusters(hl_context* c, const GpuCameraUniforms* 
     c->hot_src = nullptr;  // set again once the records are rebuilt
     if ((s = ensure(c, c->cull, sizeof(CullLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
     if ((s = ensure(c, c->hot, sizeof(HotLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
-    if ((s = ensure(c, c->geom, cluster_geom_bytes(ncol, (uint32_t)ncell))) != HL_OK) return s;
-    if ((s = ensure(c, c->bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
-    if ((s = ensure(c, c->summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;
     if ((s = ensure(c, c->raw, cluster_raw_bytes((uint32_t)ncell))) != HL_OK) return s;
-    if ((s = ensure(c, c->markq, mark_queue_bytes(n))) != HL_OK) return s;
+    const size_t columns = column_scratch_bytes(p->grid_x, p->grid_y, p->grid_z, n);
+    if (columns) {
+        if ((s = ensure(c, c->columns, columns)) != HL_OK) return s;
+    } else {
+        if ((s = ensure(c, c->geom, cluster_geom_bytes(ncol, (uint32_t)ncell))) != HL_OK) return s;
+        if ((s = ensure(c, c->bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
+        if ((s = ensure(c, c->summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;
+        if ((s = ensure(c, c->markq, mark_queue_bytes(n))) != HL_OK) return s;
+    }
     HL_HIP(c, hipSetDevice(c->device));
     // the overflow word(s) are reset by the first cull kernel and OR-ed by the
     // list kernel: the caller's word when given, and always the context's copy
@@ -642,7 +647,7 @@ HL_API hl_status hl_light_cull_clusters(hl_context* c, const GpuCameraUniforms* 
     uint32_t* flags2 = overflow_d ? ctx_words(c) : nullptr;
     ClusterArgs a = make_cluster_args(p, n);
     ClusterScratch w{c->geom.p, (uint32_t*)c->bits.p, (uint32_t*)c->summary.p, (uint32_t*)c->raw.p,
-                     mark_queue_at(c->markq.p, n)};
+                     mark_queue_at(c->markq.p, n), c->columns.p};
     HL_HIP(c, launch_cluster_cull(c->stream, a, camera_d, lights_d, (HotLight*)c->hot.p, (CullLight*)c->cull.p,
                                   ctx_words(c) + 1, w, offsets_d, counts_d, pool_d, pool_cap, flags, flags2));
     c->hot_src = lights_d;

@@ -6,6 +6,7 @@
 //  k_cluster_geom     per column: NDC rectangle and lateral planes; per cell:
 //                     the view-space AABB; its blocks past the cells prepare
 //                     the lights (as k_prep_lights) in the same launch
+//                     (this and the next four: grids past the column path's)
 //  k_cluster_mark     light-parallel: each light bounds the cells it can reach
 //                     (projected bounding box x slice range); a wavefront tests
 //                     those candidates 64 at a time with the exact membership
@@ -19,9 +20,13 @@
 //                     sums and the counts before it (the exclusive scan, no
 //                     separate launch), then the ascending indices from the
 //                     bitmask, which it clears again for the next call
+//  k_col_*            the clustered lists a column of the grid per block (most
+//                     grids; see the section)
 //  k_batch_*          the same steps for many views in one launch each
 // Membership is decided by the same exact FP32 tests whatever the order of
 // evaluation, so the lists equal the per-cluster brute force bit for bit.
+#include <algorithm>
+
 #include "hl_internal.hpp"
 
 namespace hl {
@@ -292,6 +297,38 @@ struct MarkBox {
     uint32_t x0, y0, s0, nx, ny, nz;
 };
 
+// The columns of that bound for a light in front of the camera (centre c,
+// view distance zc > 0, widened radius rr; p00, p11 > 0), before clamping to
+// the grid: inclusive x and y ranges, each end in [-1, grid].
+__device__ __forceinline__ void light_columns(const ClusterArgs& a, float p00, float p11, float4 c, float zc,
+                                              float rr, int* x0, int* x1, int* y0, int* y1) {
+    const int gx = (int)a.grid_x, gy = (int)a.grid_y;
+    const float fx = __builtin_amdgcn_sqrtf(1.0f + hl_f_rcp(p00 * p00));
+    const float fy = __builtin_amdgcn_sqrtf(1.0f + hl_f_rcp(p11 * p11));
+    const float iz = hl_f_rcp(zc);
+    const float nx0 = p00 * (c.x - rr * fx) * iz, nx1 = p00 * (c.x + rr * fx) * iz;
+    const float ny0 = p11 * (c.y - rr * fy) * iz, ny1 = p11 * (c.y + rr * fy) * iz;
+    const float fw = (float)a.width, fh = (float)a.height;
+    float px0 = (nx0 + 1.0f) * 0.5f * fw, px1 = (nx1 + 1.0f) * 0.5f * fw;
+    float py0 = (1.0f - ny1) * 0.5f * fh, py1 = (1.0f - ny0) * 0.5f * fh;
+    px0 -= 1e-5f * fabsf(px0) + 0.25f;
+    px1 += 1e-5f * fabsf(px1) + 0.25f;
+    py0 -= 1e-5f * fabsf(py0) + 0.25f;
+    py1 += 1e-5f * fabsf(py1) + 0.25f;
+    const float icw = hl_f_rcp((float)a.cell_w), ich = hl_f_rcp((float)a.cell_h);
+    // clamped to [-1, g] before the conversion (NaN: the whole range)
+    *x0 = (int)fminf(fmaxf(floorf(px0 * icw), -1.0f), (float)gx);
+    *x1 = (int)fmaxf(fminf(floorf(px1 * icw), (float)gx), -1.0f);
+    *y0 = (int)fminf(fmaxf(floorf(py0 * ich), -1.0f), (float)gy);
+    *y1 = (int)fmaxf(fminf(floorf(py1 * ich), (float)gy), -1.0f);
+}
+
+// Whether a light's cells can be bounded at all (else: the whole grid).
+__device__ __forceinline__ bool light_bounded(float4 vpos) {
+    return !__builtin_isinf(vpos.w) && __builtin_isfinite(-vpos.z) && __builtin_isfinite(vpos.x) &&
+           __builtin_isfinite(vpos.y);
+}
+
 // All 64 lanes must be active (the slice limits are found by ballots); sp is
 // slice_r_pad[lane] (lanes below grid_z; slice_near, slice_far and the
 // paddings are non-decreasing, checked by the host).
@@ -305,8 +342,7 @@ __device__ __forceinline__ bool light_cells(const ClusterArgs& a,
     const float sn = vn - 1e-5f * fabsf(vn), sf = vf + 1e-5f * fabsf(vf);
     int x0 = 0, x1 = gx - 1, y0 = 0, y1 = gy - 1, s0 = 0, s1 = gz - 1;
     const float zc = -L.vpos.z;
-    if (!__builtin_isinf(L.vpos.w) && __builtin_isfinite(zc) && __builtin_isfinite(L.vpos.x) &&
-        __builtin_isfinite(L.vpos.y)) {
+    if (light_bounded(L.vpos)) {
         const float slack = 1e-5f * (fabsf(L.vpos.x) + fabsf(L.vpos.y) + fabsf(zc));
         const float r = fabsf(L.vpos.w);
         // slices in reach under the largest padding, then under the largest
@@ -318,26 +354,8 @@ __device__ __forceinline__ bool light_cells(const ClusterArgs& a,
         s0 = (int)__popcll(hl_ballot(sl && sf < zc - rr));
         s1 = (int)__popcll(hl_ballot(sl && sn <= zc + rr)) - 1;
         const float p00 = cam->proj[0], p11 = cam->proj[5];
-        if (zc > 1e-4f && p00 > 0.0f && p11 > 0.0f) {
-            const float fx = __builtin_amdgcn_sqrtf(1.0f + hl_f_rcp(p00 * p00));
-            const float fy = __builtin_amdgcn_sqrtf(1.0f + hl_f_rcp(p11 * p11));
-            const float iz = hl_f_rcp(zc);
-            const float nx0 = p00 * (L.vpos.x - rr * fx) * iz, nx1 = p00 * (L.vpos.x + rr * fx) * iz;
-            const float ny0 = p11 * (L.vpos.y - rr * fy) * iz, ny1 = p11 * (L.vpos.y + rr * fy) * iz;
-            const float fw = (float)a.width, fh = (float)a.height;
-            float px0 = (nx0 + 1.0f) * 0.5f * fw, px1 = (nx1 + 1.0f) * 0.5f * fw;
-            float py0 = (1.0f - ny1) * 0.5f * fh, py1 = (1.0f - ny0) * 0.5f * fh;
-            px0 -= 1e-5f * fabsf(px0) + 0.25f;
-            px1 += 1e-5f * fabsf(px1) + 0.25f;
-            py0 -= 1e-5f * fabsf(py0) + 0.25f;
-            py1 += 1e-5f * fabsf(py1) + 0.25f;
-            const float icw = hl_f_rcp((float)a.cell_w), ich = hl_f_rcp((float)a.cell_h);
-            // clamped to [-1, g] before the conversion (NaN: the whole range)
-            x0 = (int)fminf(fmaxf(floorf(px0 * icw), -1.0f), (float)gx);
-            x1 = (int)fmaxf(fminf(floorf(px1 * icw), (float)gx), -1.0f);
-            y0 = (int)fminf(fmaxf(floorf(py0 * ich), -1.0f), (float)gy);
-            y1 = (int)fmaxf(fminf(floorf(py1 * ich), (float)gy), -1.0f);
-        }
+        if (zc > 1e-4f && p00 > 0.0f && p11 > 0.0f)
+            light_columns(a, p00, p11, L.vpos, zc, rr, &x0, &x1, &y0, &y1);
     }
     x0 = clampi(x0, 0, gx - 1);
     x1 = clampi(x1, -1, gx - 1);
@@ -881,151 +899,671 @@ __device__ __forceinline__ CellBox* view_boxes(const BatchCullView& v) {
     return (CellBox*)((uint8_t*)v.geom + cluster_geom_offset_boxes_dev(v.ca.grid_x * v.ca.grid_y));
 }
 
-// ------------------------------------------------- clusters, brute force
-// Small problems (cells x lights <= kBruteTests) take two launches instead of
-// the light-parallel chain: every cell tests every light with the membership
-// rule (cell_member), one wave per cell and four cells per block, the
-// lights' culling records built per block into LDS kBfLights at a time, each
-// cell's records built by its own wave in registers.  k_cluster_bf_count
-// stores each cell's member count (and the lights' shading records);
-// k_cluster_bf_fill finds each cell's offset from the capped counts before
-// it, then writes the ascending list.  Membership does not depend on the
-// order of evaluation, so the lists are the light-parallel path's.
-constexpr uint64_t kBruteTests = 1ull << 22;
-constexpr uint32_t kBfCells = 4;  // one per wave
-constexpr uint32_t kBfLights = 256;
+// --------------------------------------------- clusters, column by column
+// The path of every grid that use_columns accepts.  A block owns one column of
+// the grid, or kb slices of it when there are few columns (column_plan aims at
+// kColBlocks blocks, two to three per CU):
+//   k_col_prep   one thread per light: its shading and culling records and
+//                its candidate box (light_box: the mark path's bound, packed
+//                into 8 bytes);
+//   k_col_count  scans the boxes (a compare each) into a bit per candidate
+//                light, lists the candidates in LDS in ascending order, tests
+//                each one (a lane) against the slices of its box with the
+//                membership rule -- the four plane distances once per
+//                candidate, as they do not depend on the slice -- and stores
+//                the candidates with a bit per member slice, and the counts;
+//   k_col_fill   the exclusive prefix of the capped counts, and the lists: the
+//                candidates' slice bits transposed into a bit per (slice,
+//                candidate) in LDS, each word of which a thread expands.
+// Small problems (column_inline) skip k_col_prep: every count block bounds
+// all lights itself, which costs less than a launch.
+// Nothing is written per (cell, light): the bitmask over cells and lights of
+// the mark path (57 MB at 32x18x48 cells and 16384 lights, two atomics per
+// member) is not touched, and the geometry of a column lives in its block's
+// LDS.  What bounds it is latency: the barriers and memory round trips of one
+// block's chain, the fullest columns' (1200 candidates at 4K) above all.
+// Measured (kernel times, us): 32x18x48 cells and 16384 lights 32 (prep 6.6,
+// count 14.6, fill 10.7) against the mark path's 52 (geometry 5.8, mark 14.7,
+// tail 4.5, count 10.5, fill 16.1); 16x9x24 and 1024 lights 21 against 50 for
+// two brute-force launches, 256 lights 15 against 23.  1000 blocks aimed at
+// instead of 512 made the 4K count 18.8.
+constexpr uint32_t kColMaxColumns = 2048;
+constexpr uint32_t kColBlocks = 512;
+constexpr uint32_t kColChunk = 16384;  // lights scanned at a time
+constexpr uint32_t kColThreads = 512;  // of a count block
+constexpr uint32_t kColInline = 512;   // lights every block bounds itself
+constexpr uint32_t kColInlineCells = 8192;
+constexpr uint32_t kColBatch = 512;    // candidates a fill block lists at a time
+constexpr uint32_t kColGroup = 16;     // columns per partial sum of counts
 
-struct BfSmem {
-    CullLight light[kBfLights];
-    uint32_t capped[kBfCells];
-    unsigned long long part[4];
-    uint32_t flags;
+// A light's candidate cells (inclusive ranges).  col: its columns, a byte each
+// for x0, y0, 127 - x1 and 127 - y1 (grids of at most 128 columns a side), so
+// that one subtraction holds a column against all four ends; slice: s0 | s1 << 8,
+// the top bit set for a light with a cone test.
+struct LightBox {
+    uint32_t col, slice;
+};
+constexpr uint32_t kNoBox = 0x7F7F7F7Fu;  // x >= 127 and x <= 0
+constexpr uint32_t kBoxCone = 0x80000000u;
+constexpr uint32_t kColMaxSide = 128;
+__device__ __forceinline__ uint32_t box_s0(uint32_t s) { return s & 0xFFu; }
+__device__ __forceinline__ uint32_t box_s1(uint32_t s) { return (s >> 8) & 0xFFu; }
+
+// Sums of counts fit in 32 bits: use_columns keeps cells x lights at 2^31.
+struct ColumnArgs {
+    const GpuCameraUniforms* cam;
+    const GpuLight* lights;
+    const uint32_t* subset;   // pool indices of the lights, or null
+    HotLight* hot;
+    CullLight* cull;          // per light (k_col_prep)
+    uint32_t* box_col;        // LightBox::col per light, to a multiple of four (k_col_prep)
+    uint32_t* box_slice;      // LightBox::slice per light (k_col_prep)
+    uint32_t* feature_flags;
+    uint32_t* num_cand;       // per block
+    uint64_t* cand_slices;    // per block and candidate (n per block): its member slices, bit k: slice k0 + k
+    uint32_t* cand;           // the candidate's light
+    uint32_t* gsum;           // capped counts per (slice, group of columns) (k_col_prep)
+    uint32_t* raw;            // per cell: members before the cap
+    uint32_t* offsets;
+    uint32_t* counts;
+    uint32_t* pool;
+    uint32_t pool_cap;
+    uint32_t kb;              // slices per block
+    uint32_t* flags;
+    uint32_t* flags2;
 };
 
-// The records of the wave's cell (every lane alike).
-struct BfCell {
-    ColumnGeom g;
-    CellBox bx;
-    float pad;
+// The slice tables as the candidate bound reads them: the near and far
+// distances rounded outwards, and the paddings.
+struct SliceTab {
+    float sn[HL_MAX_SLICES], sf[HL_MAX_SLICES], pad[HL_MAX_SLICES];
 };
-__device__ __forceinline__ BfCell bf_cell(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
-                                          uint32_t cell, uint32_t ncell) {
-    BfCell c;
-    const uint32_t ncol = a.grid_x * a.grid_y;
-    if (cell < ncell) {
-        cell_geometry(a, cam, cell % ncol, cell / ncol, true, c.g, c.bx);
-        c.pad = a.slice_r_pad[cell / ncol];
-    } else {  // no cell: no member (the records are not read)
-        c.g = ColumnGeom{};
-        c.bx = CellBox{};
-        c.pad = 0.0f;
+__device__ __forceinline__ void load_slices(const ClusterArgs& a, SliceTab& t) {
+    const uint32_t k = threadIdx.x;
+    if (k < a.grid_z) {
+        const float vn = a.slice_near[k], vf = a.slice_far[k];
+        t.sn[k] = vn - 1e-5f * fabsf(vn);
+        t.sf[k] = vf + 1e-5f * fabsf(vf);
+        t.pad[k] = a.slice_r_pad[k];
     }
+}
+
+// Entries of the ascending table v[0, n) that are <= x, or < x (n <= 64).
+template <bool kStrict>
+__device__ __forceinline__ int count_below(const float* v, int n, float x) {
+    int k = 0;
+#pragma unroll
+    for (int step = 64; step; step >>= 1) {
+        const int j = k + step;
+        if (j <= n && (kStrict ? v[j - 1] < x : v[j - 1] <= x)) k = j;
+    }
+    return k;
+}
+
+// light_cells for one thread, the slice limits by bisection.
+__device__ __forceinline__ LightBox light_box(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
+                                           float4 vpos, bool cone, const SliceTab& t) {
+    const int gx = (int)a.grid_x, gy = (int)a.grid_y, gz = (int)a.grid_z;
+    int x0 = 0, x1 = gx - 1, y0 = 0, y1 = gy - 1, s0 = 0, s1 = gz - 1;
+    const LightBox none{kNoBox, 0u};
+    if (light_bounded(vpos)) {
+        const float zc = -vpos.z;
+        const float slack = 1e-5f * (fabsf(vpos.x) + fabsf(vpos.y) + fabsf(zc));
+        const float r = fabsf(vpos.w);
+        float rr = (r + t.pad[gz - 1]) * (1.0f + 1e-5f) + slack;
+        s1 = count_below<false>(t.sn, gz, zc + rr) - 1;
+        if (s1 < 0) return none;
+        rr = (r + t.pad[s1]) * (1.0f + 1e-5f) + slack;
+        s0 = count_below<true>(t.sf, gz, zc - rr);
+        while (s1 >= 0 && !(t.sn[s1] <= zc + rr)) --s1;  // seldom any: rr only shrank
+        const float p00 = cam->proj[0], p11 = cam->proj[5];
+        if (zc > 1e-4f && p00 > 0.0f && p11 > 0.0f)
+            light_columns(a, p00, p11, vpos, zc, rr, &x0, &x1, &y0, &y1);
+    }
+    x0 = clampi(x0, 0, gx - 1);
+    x1 = clampi(x1, -1, gx - 1);
+    y0 = clampi(y0, 0, gy - 1);
+    y1 = clampi(y1, -1, gy - 1);
+    s0 = clampi(s0, 0, gz - 1);
+    s1 = clampi(s1, -1, gz - 1);
+    if (x1 < x0 || y1 < y0 || s1 < s0) return none;
+    return LightBox{(uint32_t)x0 | (uint32_t)y0 << 8 | (uint32_t)(127 - x1) << 16 | (uint32_t)(127 - y1) << 24,
+                    (uint32_t)s0 | (uint32_t)s1 << 8 | (cone ? kBoxCone : 0u)};
+}
+
+// Whether the box holds a column, given as column_key: every byte of the key
+// (with its top bit as a guard) at least the box's.
+constexpr uint32_t kByteTops = 0x80808080u;
+__device__ __forceinline__ uint32_t column_key(uint32_t cx, uint32_t cy) {
+    return kByteTops | cx | cy << 8 | (127u - cx) << 16 | (127u - cy) << 24;
+}
+__device__ __forceinline__ bool box_has_column(uint32_t col, uint32_t key) {
+    return ((key - col) & kByteTops) == kByteTops;
+}
+__device__ __forceinline__ bool box_has_slices(uint32_t s, uint32_t k0, uint32_t k1) {
+    return box_s0(s) <= k1 && box_s1(s) >= k0;
+}
+
+// A cell's box and the padding of its slice, as two 16-byte LDS reads.
+struct alignas(16) ColCell {
+    float lo[3], hi[3], pad, unused;
+};
+struct ColGeomSmem {
+    float3 pl[4];                 // the column's planes
+    ColCell cell[HL_MAX_SLICES];  // the block's cells
+    SliceTab tab;
+};
+template <uint32_t CHUNK>
+struct ColCountSmem {
+    ColGeomSmem g;
+    uint32_t words[CHUNK / 32];  // candidate bits of the chunk
+    uint16_t list[CHUNK];        // the candidates, ascending, chunk-relative
+    uint32_t wave_sum[kColThreads / 64];
+    uint32_t cnt[kColThreads / 64][HL_MAX_SLICES];
+};
+struct ColFillSmem {
+    uint32_t bits[HL_MAX_SLICES][kColBatch / 32];  // members of the batch per slice
+    uint32_t light[kColBatch];
+    uint32_t off[HL_MAX_SLICES], cnt[HL_MAX_SLICES], run[HL_MAX_SLICES];
+    uint32_t row[HL_MAX_SLICES], part[HL_MAX_SLICES], base[4];
+};
+
+// The block's column and slices: blocks run slice group by slice group over
+// the columns.
+struct ColBlock {
+    uint32_t col, cx, cy, k0, nk, ncol;
+};
+__device__ __forceinline__ ColBlock col_block(const ClusterArgs& a, uint32_t block, uint32_t kb) {
+    ColBlock c;
+    c.ncol = a.grid_x * a.grid_y;
+    c.col = block % c.ncol;
+    c.cx = c.col % a.grid_x;
+    c.cy = c.col / a.grid_x;
+    c.k0 = block / c.ncol * kb;
+    c.nk = min(kb, a.grid_z - c.k0);
     return c;
 }
 
-// For each light of the LDS chunk [l0, l0 + kBfLights) in ascending order, in
-// groups of 64: f(group, pass) with pass this lane's light's membership in
-// the wave's cell (uniform calls).
-template <class F>
-__device__ __forceinline__ void bf_chunk(const ClusterArgs& a, uint32_t l0, const BfCell& c, const BfSmem& sm,
-                                         F&& f) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t nl = a.num_lights - l0 < kBfLights ? a.num_lights - l0 : kBfLights;
-    for (uint32_t j0 = 0; j0 < nl; j0 += 64u) {
-        const uint32_t j = j0 + lane;
-        const bool pass = c.g.on != 0u && j < nl && cell_member(sm.light[j], c.g, c.bx, c.pad);
-        f(j0, pass);
+// The planes of the column and the boxes of its cells (cell_geometry's, a
+// plane or a box per thread of the block's last two waves, which have no
+// lights to bound in the smallest problems) into LDS; the caller
+// synchronises.  Returns whether the column covers pixels (uniform).
+__device__ __forceinline__ bool col_setup(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
+                                          const ColBlock& c, ColGeomSmem& sm) {
+    const uint32_t t = threadIdx.x - (kColThreads - 64u);  // wraps: another wave
+    if (t < c.nk) {
+        ColumnGeom g;
+        CellBox bx;
+        cell_geometry(a, cam, c.col, c.k0 + t, false, g, bx);
+        ColCell& o = sm.cell[t];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            o.lo[i] = bx.lo[i];
+            o.hi[i] = bx.hi[i];
+        }
+        o.pad = a.slice_r_pad[c.k0 + t];
     }
+    float l = 0.0f, r = 0.0f, b = 0.0f, tp = 0.0f;
+    const bool on = column_rect(a, c.cx, c.cy, &l, &r, &b, &tp);
+    const uint32_t p = threadIdx.x - (kColThreads - 128u);
+    if (on && p < 4u) {
+        // (l, b, l, t), (r, t, r, b), (l, t, r, t), (r, b, l, b)
+        const float x0 = (p == 0u || p == 2u) ? l : r, y0 = (p == 0u || p == 3u) ? b : tp;
+        const float x1 = (p == 0u || p == 3u) ? l : r, y1 = (p == 0u || p == 2u) ? tp : b;
+        sm.pl[p] = hl_x_plane(cam->proj[0], cam->proj[5], x0, y0, x1, y1);
+    }
+    return on;
 }
 
-__device__ __forceinline__ void bf_load_lights(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
-                                               const GpuLight* __restrict__ lights, uint32_t l0, BfSmem& sm) {
-    __syncthreads();  // the previous chunk is no longer read
-    const uint32_t i = l0 + threadIdx.x;
-    if (i < a.num_lights) sm.light[threadIdx.x] = cull_light_at(lights, i, cam);
-    __syncthreads();
-}
-
-__global__ __launch_bounds__(256) void k_cluster_bf_count(ClusterArgs a, const GpuCameraUniforms* __restrict__ cam,
-                                                          const GpuLight* __restrict__ lights,
-                                                          HotLight* __restrict__ hot,
-                                                          uint32_t* __restrict__ feature_flags,
-                                                          uint32_t* __restrict__ raw, uint32_t* __restrict__ flags,
-                                                          uint32_t* __restrict__ flags2) {
-    __shared__ BfSmem sm;
-    const uint32_t ncell = a.grid_x * a.grid_y * a.grid_z;
-    const uint32_t cell = blockIdx.x * kBfCells + (threadIdx.x >> 6);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {  // OR-ed by the fill launch
-        *flags = 0u;
-        if (flags2) *flags2 = 0u;
-    }
-    // the shading records, grid-stride over the lights
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.num_lights; i += gridDim.x * blockDim.x)
-        prep_one(lights, nullptr, a.num_lights, cam, hot, nullptr, feature_flags, i);
-    const BfCell c = bf_cell(a, cam, cell, ncell);
-    uint32_t cnt = 0u;
-    for (uint32_t l0 = 0; l0 < a.num_lights; l0 += kBfLights) {
-        bf_load_lights(a, cam, lights, l0, sm);
-        bf_chunk(a, l0, c, sm, [&](uint32_t, bool pass) { cnt += (uint32_t)__popcll(hl_ballot(pass)); });
-    }
-    if ((threadIdx.x & 63u) == 0 && cell < ncell) raw[cell] = cnt;
-}
-
-__global__ __launch_bounds__(256) void k_cluster_bf_fill(ClusterArgs a, const GpuCameraUniforms* __restrict__ cam,
-                                                         const GpuLight* __restrict__ lights,
-                                                         const uint32_t* __restrict__ raw, uint32_t pool_cap,
-                                                         uint32_t* __restrict__ offsets, uint32_t* __restrict__ counts,
-                                                         uint32_t* __restrict__ pool, uint32_t* __restrict__ flags,
-                                                         uint32_t* __restrict__ flags2) {
-    __shared__ BfSmem sm;
-    const uint32_t ncell = a.grid_x * a.grid_y * a.grid_z, first = blockIdx.x * kBfCells;
+// Lists the set bits of words[0, nw) (nw <= W) in list, ascending; returns
+// their number.  Called by all NT threads; ends with the list visible to them.
+template <uint32_t W, uint32_t NT>
+__device__ __forceinline__ uint32_t list_bits(const uint32_t* words, uint32_t nw, uint16_t* list,
+                                              uint32_t* wave_sum) {
+    constexpr uint32_t kPer = (W + NT - 1u) / NT;  // words per thread
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-    const uint32_t cell = first + wave, cap = a.cap;
-    // capped counts of the cells before the block
-    unsigned long long acc = 0;
-    for (uint32_t j = t; j < first; j += blockDim.x) {
-        const uint32_t v = raw[j];
-        acc += (cap && v > cap) ? cap : v;
+    uint32_t w[kPer], n = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q) {
+        const uint32_t i = t * kPer + q;
+        w[q] = i < nw ? words[i] : 0u;
+        n += (uint32_t)__popc(w[q]);
     }
-    acc = wave_sum_u64(acc);
-    if (lane == 0) sm.part[wave] = acc;
-    if (t == 0) sm.flags = 0u;
-    if (t < kBfCells) {
-        const uint32_t v = first + t < ncell ? raw[first + t] : 0u;
-        sm.capped[t] = (cap && v > cap) ? cap : v;
+    uint32_t incl = n;
+#pragma unroll
+    for (uint32_t o = 1; o < 64u; o <<= 1) {
+        const uint32_t u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
     }
-    const BfCell c = bf_cell(a, cam, cell, ncell);
+    if (lane == 63u) wave_sum[wave] = incl;
     __syncthreads();
-    // the wave's cell: offset, count after the cap and the pool truncation
-    unsigned long long base = sm.part[0] + sm.part[1] + sm.part[2] + sm.part[3];
-    for (uint32_t j = 0; j < wave; ++j) base += sm.capped[j];
-    const uint32_t o = base > pool_cap ? pool_cap : (uint32_t)base;
-    uint32_t cnt = sm.capped[wave], fl = 0u;
-    if (cell < ncell && cap && raw[cell] > cap) fl |= HL_OVERFLOW_CAP;
-    if (cnt > pool_cap - o) {
-        cnt = pool_cap - o;
-        fl |= HL_OVERFLOW_POOL;
+    uint32_t pos = incl - n, total = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < NT / 64u; ++q) {
+        if (q < wave) pos += wave_sum[q];
+        total += wave_sum[q];
     }
-    if (lane == 0 && cell < ncell) {
-        offsets[cell] = o;
-        counts[cell] = cnt;
-        if (fl) atomicOr(&sm.flags, fl);
-    }
-    uint32_t written = 0u;
-    for (uint32_t l0 = 0; l0 < a.num_lights; l0 += kBfLights) {
-        bf_load_lights(a, cam, lights, l0, sm);
-        bf_chunk(a, l0, c, sm, [&](uint32_t j0, bool pass) {
-            const uint64_t m = hl_ballot(pass);
-            const uint32_t pos = written + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            if (pass && pos < cnt) pool[o + pos] = l0 + j0 + lane;
-            written += (uint32_t)__popcll(m);
-        });
-    }
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q)
+        for (uint32_t m = w[q]; m; m &= m - 1u)
+            list[pos++] = (uint16_t)(32u * (t * kPer + q) + (uint32_t)__builtin_ctz(m));
     __syncthreads();
-    if (t == 0 && sm.flags) {
-        atomicOr(flags, sm.flags);
-        if (flags2) atomicOr(flags2, sm.flags);
+    return total;
+}
+
+// The OR of a 64-bit word over the wave, in every lane (scalar).
+__device__ __forceinline__ uint64_t wave_or(uint64_t v) {
+    const auto red = [](uint32_t x) {
+        x |= (uint32_t)hl_dpp_i<0xB1>(0, (int)x);
+        x |= (uint32_t)hl_dpp_i<0x4E>(0, (int)x);
+        x |= (uint32_t)hl_dpp_i<0x141>(0, (int)x);
+        x |= (uint32_t)hl_dpp_i<0x140>(0, (int)x);
+        x |= (uint32_t)hl_dpp_i<0x142, 0xA>(0, (int)x);
+        x |= (uint32_t)hl_dpp_i<0x143, 0xC>(0, (int)x);
+        return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+    };
+    return (uint64_t)red((uint32_t)v) | (uint64_t)red((uint32_t)(v >> 32)) << 32;
+}
+
+// The slices [k0, k0 + nk) of the column that light L
+// (candidate slices box_slice) is a member of: the rule of cell_member.  !(d < -r) for every
+// plane is !(min d < -r): the comparison is false for a NaN distance, which
+// fminf drops.
+__device__ __forceinline__ uint64_t member_slices(const ColBlock& c, const ColGeomSmem& sm, const CullLight& L,
+                                                  uint32_t box_slice) {
+#pragma clang fp contract(off)
+    float d = __builtin_inff();
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+        d = fminf(d, hl_x_dot3(sm.pl[p].x, sm.pl[p].y, sm.pl[p].z, L.vpos.x, L.vpos.y, L.vpos.z) + 0.0f);
+    const uint32_t ka = max(box_s0(box_slice), c.k0), kz = min(box_s1(box_slice), c.k0 + c.nk - 1u);
+    uint64_t m = 0;
+    for (uint32_t k = ka; k <= kz; ++k) {
+        const float4* q = reinterpret_cast<const float4*>(&sm.cell[k - c.k0]);
+        const float4 q0 = q[0], q1 = q[1];
+        const float rc = L.vpos.w + q1.z;
+        const float3 lo = make_float3(q0.x, q0.y, q0.z), hi = make_float3(q0.w, q1.x, q1.y);
+        bool in = !(d < -rc) && hl_x_sphere_aabb(L.vpos, rc, lo, hi);
+        if (in && (box_slice & kBoxCone)) in = hl_x_cone_cell(L.vpos, L.axis, L.aux.x, q1.z, lo, hi);
+        if (in) m |= 1ull << (k - c.k0);
     }
+    return m;
+}
+
+// A wave per block: the lights' chains (loads, FP64 band, bisections) over all
+// CUs rather than over n / 256 of them.
+__global__ __launch_bounds__(64) void k_col_prep(ClusterArgs a, ColumnArgs p, uint32_t nsum) {
+    __shared__ SliceTab tab;
+    load_slices(a, tab);
+    __syncthreads();
+    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+    if (i == 0) {
+        *p.flags = 0u;
+        if (p.flags2) *p.flags2 = 0u;
+    }
+    for (uint32_t j = i; j < nsum; j += gridDim.x * 64u) p.gsum[j] = 0u;
+    if (i >= a.num_lights) {
+        if (i < ((a.num_lights + 3u) & ~3u)) p.box_col[i] = kNoBox;
+        return;
+    }
+    const CullLight L = cull_light_at(p.lights, i, p.cam);
+    p.cull[i] = L;
+    const LightBox b = light_box(a, p.cam, L.vpos, L.cone.w != kNoCone, tab);
+    p.box_col[i] = b.col;
+    p.box_slice[i] = b.slice;
+    prep_one(p.lights, nullptr, a.num_lights, p.cam, p.hot, nullptr, p.feature_flags, i);
+}
+
+// INLINE: the block bounds every light itself (a light per thread; the cone
+// terms come with the candidate's record), and the blocks share the shading
+// records.
+template <uint32_t CHUNK, bool INLINE>
+__device__ __forceinline__ void col_count_block(const ClusterArgs& a, const ColumnArgs& p, uint32_t block,
+                                                uint32_t nblocks, ColCountSmem<CHUNK>& sm, uint32_t* inline_slices) {
+    constexpr uint32_t NT = kColThreads, kWaves = NT / 64u;
+    static_assert(!INLINE || CHUNK == NT, "a light per thread");
+    constexpr uint32_t kAhead = 8u;  // loads of four lights' columns in flight per lane
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, n = a.num_lights;
+    const ColBlock c = col_block(a, block, p.kb);
+    float4 pr = make_float4(0.0f, 0.0f, 0.0f, 0.0f), dro = pr;
+    uint32_t type = 0u;
+    if (INLINE && t < n) {  // in flight during the set-up
+        pr = *reinterpret_cast<const float4*>(p.lights[t].position_range);
+        dro = *reinterpret_cast<const float4*>(p.lights[t].direction_outer);
+        type = p.lights[t].light_type;
+    }
+    if (INLINE) {  // the bounds read the slice tables
+        load_slices(a, sm.g.tab);
+        __syncthreads();
+    }
+    const bool on = col_setup(a, p.cam, c, sm.g);
+    const uint32_t key = column_key(c.cx, c.cy), k1 = c.k0 + c.nk - 1u;
+    [[maybe_unused]] const bool part_column = c.nk != a.grid_z;
+    if (INLINE && block == 0 && t == 0) {
+        *p.flags = 0u;
+        if (p.flags2) *p.flags2 = 0u;
+    }
+    uint32_t cnt = 0;  // lane k: members of slice k0 + k among the wave's candidates
+    uint32_t done = 0;
+    uint32_t* const cand = p.cand + (size_t)block * n;
+    uint64_t* const cand_slices = p.cand_slices + (size_t)block * n;
+    for (uint32_t l0 = 0; l0 < n; l0 += CHUNK) {
+        const uint32_t nl = min(CHUNK, n - l0), nw = (nl + 31u) / 32u;
+        if (l0) __syncthreads();  // the previous chunk's list is no longer read
+        if (INLINE) {
+            bool m = false;
+            if (t < n) {
+                const float* v = p.cam->view;
+                const float4 vp = make_float4(hl_x_mat_row(v, 0, pr.x, pr.y, pr.z, 1.0f),
+                                              hl_x_mat_row(v, 1, pr.x, pr.y, pr.z, 1.0f),
+                                              hl_x_mat_row(v, 2, pr.x, pr.y, pr.z, 1.0f),
+                                              type == HL_LIGHT_DIRECTIONAL ? __builtin_inff() : pr.w);
+                const LightBox b = light_box(a, p.cam, vp, type == HL_LIGHT_SPOT, sm.g.tab);
+                inline_slices[t] = b.slice;
+                m = on && box_has_column(b.col, key) && box_has_slices(b.slice, c.k0, k1);
+            }
+            const uint64_t bal = hl_ballot(m);
+            if (lane < 2u) sm.words[2u * wave + lane] = lane ? (uint32_t)(bal >> 32) : (uint32_t)bal;
+        } else {
+            // a lane takes 4 kAhead lights at a time, their columns loaded
+            // together, and sets the bits of the few that hold its column;
+            // blocks start at different lights, so that they do not all read
+            // the same lines at the same time
+            for (uint32_t w = t; w < nw; w += NT) sm.words[w] = 0u;
+            __syncthreads();
+            const uint4* cols = reinterpret_cast<const uint4*>(p.box_col + l0);
+            const uint32_t quads = (nl + 3u) / 4u, groups = (quads + NT - 1u) / NT, rot = block % groups;
+            for (uint32_t g0 = 0; g0 < groups; g0 += kAhead) {
+                uint4 v[kAhead];
+#pragma unroll
+                for (uint32_t q = 0; q < kAhead; ++q) {
+                    const uint32_t g = g0 + q + rot, j = (g < groups ? g : g - groups) * NT + t;
+                    v[q] = make_uint4(kNoBox, kNoBox, kNoBox, kNoBox);
+                    if (g0 + q < groups && j < quads) v[q] = cols[j];
+                }
+                uint32_t hits = 0;
+#pragma unroll
+                for (uint32_t q = 0; q < kAhead; ++q) {
+                    hits |= box_has_column(v[q].x, key) ? 1u << (4u * q) : 0u;
+                    hits |= box_has_column(v[q].y, key) ? 2u << (4u * q) : 0u;
+                    hits |= box_has_column(v[q].z, key) ? 4u << (4u * q) : 0u;
+                    hits |= box_has_column(v[q].w, key) ? 8u << (4u * q) : 0u;
+                }
+                for (; hits && on; hits &= hits - 1u) {
+                    const uint32_t b = (uint32_t)__builtin_ctz(hits), g = g0 + (b >> 2) + rot;
+                    const uint32_t j = 4u * ((g < groups ? g : g - groups) * NT + t) + (b & 3u);
+                    if (part_column && !box_has_slices(p.box_slice[l0 + j], c.k0, k1)) continue;
+                    atomicOr(&sm.words[j >> 5], 1u << (j & 31u));
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t total = list_bits<CHUNK / 32u, NT>(sm.words, nw, sm.list, sm.wave_sum);
+        for (uint32_t j0 = 0; j0 + wave * 64u < total; j0 += NT) {  // uniform over the wave
+            const uint32_t j = j0 + t;
+            uint64_t m = 0;
+            if (j < total) {
+                const uint32_t r = sm.list[j], li = l0 + r;
+                CullLight L;
+                uint32_t slice;
+                if (INLINE) {
+                    slice = inline_slices[r];
+                    L = cull_light_at(p.lights, r, p.cam);
+                    if (L.cone.w == kNoCone) slice &= ~kBoxCone;
+                } else {
+                    const CullLight* cl = p.cull + li;
+                    slice = p.box_slice[li];
+                    L.vpos = hl_ld4(&cl->vpos);
+                    L.axis = L.aux = L.vpos;
+                    if (slice & kBoxCone) {
+                        L.axis = hl_ld4(&cl->axis);
+                        L.aux.x = cl->aux.x;
+                    }
+                }
+                m = member_slices(c, sm.g, L, slice);
+                cand[done + j] = li;
+                cand_slices[done + j] = m;
+            }
+            // the slices that some candidate of the wave is a member of
+            for (uint64_t any = wave_or(m); any; any &= any - 1ull) {
+                const uint32_t k = (uint32_t)__builtin_ctzll(any);
+                const uint32_t members = (uint32_t)__popcll(hl_ballot((m >> k) & 1ull));
+                cnt += lane == k ? members : 0u;
+            }
+        }
+        done += total;
+    }
+    sm.cnt[wave][lane] = cnt;
+    __syncthreads();
+    if (t < c.nk) {
+        uint32_t v = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kWaves; ++w) v += sm.cnt[w][t];
+        p.raw[c.col + c.ncol * (c.k0 + t)] = v;
+        const uint32_t capped = (a.cap && v > a.cap) ? a.cap : v;
+        if (!INLINE && capped)
+            atomicAdd(p.gsum + (size_t)(c.k0 + t) * ((c.ncol + kColGroup - 1u) / kColGroup) + c.col / kColGroup, capped);
+    }
+    if (t == 0u) p.num_cand[block] = done;
+    // the shading records, last: no wait stands on them
+    if (INLINE)
+        for (uint32_t i = block * NT + t; i < n; i += nblocks * NT)
+            prep_one(p.lights, nullptr, n, p.cam, p.hot, nullptr, p.feature_flags, i);
+}
+
+// Sum over the aligned groups of 2^lp consecutive lanes.
+__device__ __forceinline__ uint32_t part_sum(uint32_t v, uint32_t lp) {
+    for (uint32_t o = 1; o < (1u << lp); o <<= 1) v += __shfl_xor(v, (int)o, 64);
+    return v;
+}
+
+// SUMS: the counts before the block's cells come from the partial sums of
+// kColGroup columns and the counts of the column's own group, else from the
+// counts of every cell before them.  A thread sums a share of one slice's
+// row (256 threads over the block's slices); those loads, the cells' own
+// counts and the first candidates go out together.
+template <bool SUMS>
+__device__ __forceinline__ void col_fill_block(const ClusterArgs& a, const ColumnArgs& p, uint32_t block,
+                                               ColFillSmem& sm) {
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, n = a.num_lights, cap = a.cap;
+    const ColBlock c = col_block(a, block, p.kb);
+    const auto capped = [&](uint32_t v) { return (cap && v > cap) ? cap : v; };
+    const uint32_t* const cand = p.cand + (size_t)block * n;
+    const uint64_t* const cand_slices = p.cand_slices + (size_t)block * n;
+    const uint32_t total = hl_uniform(p.num_cand[block]);
+    const uint32_t own = t < c.nk ? p.raw[c.col + c.ncol * (c.k0 + t)] : 0u;
+    uint32_t li[2] = {0u, 0u};
+    uint64_t ms[2] = {0ull, 0ull};
+    const auto load = [&](uint32_t b0) {
+#pragma unroll
+        for (uint32_t q = 0; q < 2u; ++q) {
+            const uint32_t j = b0 + 256u * q + t;
+            ms[q] = 0ull;
+            if (j < total) {
+                li[q] = cand[j];
+                ms[q] = cand_slices[j];
+            }
+        }
+    };
+    load(0u);
+    // rows before the block's first slice
+    const uint32_t ngrp = (c.ncol + kColGroup - 1u) / kColGroup, grp = c.col / kColGroup;
+    uint32_t acc = 0;
+    if (SUMS) {
+#pragma unroll 4
+        for (uint32_t i = t; i < c.k0 * ngrp; i += 256u) acc += p.gsum[i];
+    } else {
+#pragma unroll 8
+        for (uint32_t i = t; i < c.k0 * c.ncol; i += 256u) acc += capped(p.raw[i]);
+    }
+    // the block's rows: 2^lp threads (at most a wave) per row
+    uint32_t lp = 2;
+    while (lp < 6u && (c.nk << (lp + 1u)) <= 256u) ++lp;
+    const uint32_t k = t >> lp, part = t & ((1u << lp) - 1u);
+    uint32_t row = 0, before = 0;
+    if (k < c.nk) {
+        const size_t r = c.k0 + k;
+        if (SUMS) {
+#pragma unroll 4
+            for (uint32_t g = part; g < ngrp; g += 1u << lp) {
+                const uint32_t v = p.gsum[r * ngrp + g];
+                row += v;
+                before += g < grp ? v : 0u;
+            }
+            for (uint32_t i = grp * kColGroup + part; i < c.col; i += 1u << lp) before += capped(p.raw[r * c.ncol + i]);
+        } else {
+#pragma unroll 4
+            for (uint32_t i = part; i < c.ncol; i += 1u << lp) {
+                const uint32_t v = capped(p.raw[r * c.ncol + i]);
+                row += v;
+                before += i < c.col ? v : 0u;
+            }
+        }
+    }
+    if (c.k0) acc = part_sum(acc, 6u);
+    row = part_sum(row, lp);
+    before = part_sum(before, lp);
+    if (lane == 0u) sm.base[wave] = acc;
+    if (k < c.nk && part == 0u) {
+        sm.row[k] = row;
+        sm.part[k] = before;
+    }
+    for (uint32_t i = t; i < c.nk * (kColBatch / 32u); i += 256u) sm.bits[0][i] = 0u;
+    __syncthreads();
+    if (t < 64u) {  // the block's slices: at most 64
+        const uint32_t v = t < c.nk ? sm.row[t] : 0u;
+        uint32_t incl = v;
+#pragma unroll
+        for (uint32_t o = 1; o < 64u; o <<= 1) {
+            const uint32_t u = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += u;
+        }
+        uint32_t fl = 0u;
+        if (t < c.nk) {
+            const uint32_t off = sm.base[0] + sm.base[1] + sm.base[2] + sm.base[3] + incl - v + sm.part[t];
+            const uint32_t cell = c.col + c.ncol * (c.k0 + t);
+            uint32_t cnt = capped(own);
+            fl = cap && own > cap ? HL_OVERFLOW_CAP : 0u;
+            const uint32_t o = off > p.pool_cap ? p.pool_cap : off;
+            if (cnt > p.pool_cap - o) {
+                cnt = p.pool_cap - o;
+                fl |= HL_OVERFLOW_POOL;
+            }
+            p.offsets[cell] = o;
+            p.counts[cell] = cnt;
+            sm.off[t] = o;
+            sm.cnt[t] = cnt;
+            sm.run[t] = 0u;
+        }
+        const uint32_t any = (hl_ballot(fl & HL_OVERFLOW_CAP) ? HL_OVERFLOW_CAP : 0u) |
+                             (hl_ballot(fl & HL_OVERFLOW_POOL) ? HL_OVERFLOW_POOL : 0u);
+        if (any && t == 0u) {
+            atomicOr(p.flags, any);
+            if (p.flags2) atomicOr(p.flags2, any);
+        }
+    }
+    for (uint32_t b0 = 0; b0 < total; b0 += kColBatch) {
+        // the candidates' slice bits, transposed
+#pragma unroll
+        for (uint32_t q = 0; q < 2u; ++q) {
+            const uint32_t j = 256u * q + t;
+            sm.light[j] = li[q];
+            for (uint64_t m = ms[q]; m; m &= m - 1ull)
+                atomicOr(&sm.bits[__builtin_ctzll(m)][j >> 5], 1u << (j & 31u));
+        }
+        if (b0 + kColBatch < total) load(b0 + kColBatch);  // the next batch's, in flight meanwhile
+        __syncthreads();
+        // a thread per word, 16 lanes per slice
+        static_assert(kColBatch == 512, "16 words per slice, two candidates per thread");
+        for (uint32_t i = t; i < ((c.nk * 16u + 255u) & ~255u); i += 256u) {
+            const uint32_t s = i >> 4, w = i & 15u;
+            const bool on = s < c.nk;
+            uint32_t m = on ? sm.bits[s][w] : 0u;
+            const uint32_t v = (uint32_t)__popc(m);
+            uint32_t incl = v;
+#pragma unroll
+            for (uint32_t o = 1; o < 16u; o <<= 1) {
+                const uint32_t u = __shfl_up(incl, o, 16);
+                if (w >= o) incl += u;
+            }
+            if (!on) continue;
+            const uint32_t run = sm.run[s], cnt = sm.cnt[s], o = sm.off[s];
+            for (uint32_t pos = run + incl - v; m && pos < cnt; ++pos, m &= m - 1u)
+                p.pool[o + pos] = sm.light[32u * w + (uint32_t)__builtin_ctz(m)];
+            sm.bits[s][w] = 0u;
+            hl_wave_sync();  // the slice's 16 lanes have read its run
+            if (w == 15u) sm.run[s] = run + incl;
+        }
+        __syncthreads();  // bits, lights and runs before the next batch's
+    }
+}
+
+template <uint32_t CHUNK, bool INLINE>
+__global__ __launch_bounds__(kColThreads) void k_col_count(ClusterArgs a, ColumnArgs p) {
+    __shared__ ColCountSmem<CHUNK> sm;
+    uint32_t* is = nullptr;
+    if constexpr (INLINE) {
+        __shared__ uint32_t slices[CHUNK];
+        is = slices;
+    }
+    col_count_block<CHUNK, INLINE>(a, p, blockIdx.x, gridDim.x, sm, is);
+}
+
+template <bool SUMS>
+__global__ __launch_bounds__(256) void k_col_fill(ClusterArgs a, ColumnArgs p) {
+    __shared__ ColFillSmem sm;
+    col_fill_block<SUMS>(a, p, blockIdx.x, sm);
+}
+
+// Slices per block and blocks: whole columns when there are at least `aim` of
+// them, else enough groups of slices.
+struct ColumnPlan {
+    uint32_t kb, blocks;
+};
+static uint32_t column_groups(uint32_t ncol) { return (ncol + kColGroup - 1u) / kColGroup; }
+static ColumnPlan column_plan(uint32_t ncol, uint32_t gz, uint32_t aim) {
+    const uint32_t want = std::min(gz, (aim + ncol - 1u) / ncol);
+    const uint32_t kb = (gz + want - 1u) / want;
+    return ColumnPlan{kb, ncol * ((gz + kb - 1u) / kb)};
+}
+// The scan reads 4 bytes per (block, light) and the candidates take 12 bytes
+// of scratch each in the worst case: the column path up to 2048 columns (128
+// a side) and 2^25 (block, light) pairs.
+static bool use_columns(uint32_t gx, uint32_t gy, uint32_t gz, uint64_t n) {
+    const uint32_t ncol = gx * gy;
+    return gx <= kColMaxSide && gy <= kColMaxSide && ncol <= kColMaxColumns && column_plan(ncol, gz, kColBlocks).blocks * n <= (1ull << 25);
+}
+static bool column_inline(uint32_t ncell, uint32_t n) { return n <= kColInline && ncell <= kColInlineCells; }
+
+// Scratch of one view: candidate slices and lights, partial sums, candidate
+// numbers, boxes.
+static size_t column_scratch(uint8_t* base, uint32_t ncol, uint32_t gz, uint32_t n, uint32_t blocks, ColumnArgs* p) {
+    size_t o = 0;
+    const auto take = [&](size_t bytes) {
+        uint8_t* q = base + o;
+        o += (bytes + 255) & ~(size_t)255;
+        return q;
+    };
+    uint8_t* slices = take(8 * (size_t)blocks * n);
+    uint8_t* cand = take(4 * (size_t)blocks * n);
+    uint8_t* gsum = take(4 * (size_t)column_groups(ncol) * gz);
+    uint8_t* num = take(4 * (size_t)blocks);
+    uint8_t* box_col = take(4 * ((size_t)n + 3));
+    uint8_t* box_slice = take(4 * (size_t)n);
+    if (p) {
+        p->cand_slices = (uint64_t*)slices;
+        p->cand = (uint32_t*)cand;
+        p->gsum = (uint32_t*)gsum;
+        p->num_cand = (uint32_t*)num;
+        p->box_col = (uint32_t*)box_col;
+        p->box_slice = (uint32_t*)box_slice;
+    }
+    return o;
+}
+size_t column_scratch_bytes(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n) {
+    const uint32_t ncol = gx * gy;
+    if (!use_columns(gx, gy, gz, n)) return 0;
+    return column_scratch(nullptr, ncol, gz, n, column_plan(ncol, gz, kColBlocks).blocks, nullptr);
 }
 
 // Cells of every view, then (blocks past geom_blocks) the lights of every
@@ -1389,13 +1927,36 @@ hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCam
                                uint32_t* flags, uint32_t* flags2) {
     const uint32_t ncol = a.grid_x * a.grid_y;
     const uint32_t ncell = ncol * a.grid_z;
-    if ((uint64_t)ncell * a.num_lights <= kBruteTests) {
-        const uint32_t blocks = (ncell + kBfCells - 1u) / kBfCells;
-        k_cluster_bf_count<<<blocks, 256, 0, s>>>(a, cam, lights, hot, feature_flags, w.raw, flags, flags2);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        k_cluster_bf_fill<<<blocks, 256, 0, s>>>(a, cam, lights, w.raw, pool_cap, offsets, counts, pool, flags,
-                                                 flags2);
+    if (use_columns(a.grid_x, a.grid_y, a.grid_z, a.num_lights)) {
+        const ColumnPlan cp = column_plan(ncol, a.grid_z, kColBlocks);
+        ColumnArgs p{};
+        p.cam = cam;
+        p.lights = lights;
+        p.hot = hot;
+        p.cull = cl;
+        p.feature_flags = feature_flags;
+        p.raw = w.raw;
+        p.offsets = offsets;
+        p.counts = counts;
+        p.pool = pool;
+        p.pool_cap = pool_cap;
+        p.kb = cp.kb;
+        p.flags = flags;
+        p.flags2 = flags2;
+        (void)column_scratch((uint8_t*)w.columns, ncol, a.grid_z, a.num_lights, cp.blocks, &p);
+        hipError_t e;
+        if (column_inline(ncell, a.num_lights)) {
+            k_col_count<kColInline, true><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+            k_col_fill<false><<<cp.blocks, 256, 0, s>>>(a, p);
+            return hipGetLastError();
+        }
+        k_col_prep<<<a.num_lights ? (a.num_lights + 63u) / 64u : 1u, 64, 0, s>>>(
+            a, p, column_groups(ncol) * a.grid_z);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        k_col_count<kColChunk, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        k_col_fill<true><<<cp.blocks, 256, 0, s>>>(a, p);
         return hipGetLastError();
     }
     const uint32_t W = (a.num_lights + 31u) / 32u, SW = (W + 31u) / 32u;

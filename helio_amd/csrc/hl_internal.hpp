@@ -36,7 +36,7 @@ struct hl_context {
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
-    DevBuf hot, cull, geom, bits, summary, raw, markq, shadeq, words, accum, vogel, rcirr, tilebin;
+    DevBuf hot, cull, geom, bits, summary, raw, markq, columns, shadeq, words, accum, vogel, rcirr, tilebin;
     bool vogel_ready = false;  // vogel holds the Vogel disk tables
     // this device's address of the no-alloc scratch array (hl_api.hip),
     // looked up once per device when the context is created
@@ -155,7 +155,11 @@ struct ClusterScratch {
     uint32_t* summary;
     uint32_t* raw;       // cluster_raw_bytes(ncell)
     MarkQueue mq;        // mark_queue_bytes(lights)
+    void* columns;       // column_scratch_bytes(columns, slices, lights)
 };
+// Scratch of the column path of the clustered cull; 0: the grid and the lights
+// take the mark path (which alone needs geom, bits, summary and mq).
+size_t column_scratch_bytes(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t num_lights);
 size_t cluster_geom_bytes(uint32_t ncol, uint32_t ncell);
 size_t cluster_geom_offset_boxes(uint32_t ncol);
 inline size_t cluster_bits_words(uint32_t ncell, uint32_t num_lights) {
