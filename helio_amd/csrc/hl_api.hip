@@ -583,33 +583,23 @@ HL_API hl_status hl_light_cull_tiles(hl_context* c, const GpuCameraUniforms* cam
     if (params->screen_width == 0 || params->screen_height == 0)
         return fail(c, HL_EINVAL, "zero screen size");
     c->hot_src = nullptr;  // set again once the records are rebuilt
-    hl_status s = ensure(c, c->cull, sizeof(CullLight) * (size_t)params->num_lights);
-    if (s != HL_OK) return s;
-    if ((s = ensure(c, c->hot, sizeof(HotLight) * (size_t)params->num_lights)) != HL_OK) return s;
-    HL_HIP(c, launch_prep(c->stream, lights_d, nullptr, params->num_lights, camera_d,
-                          (HotLight*)c->hot.p, (CullLight*)c->cull.p, ctx_words(c) + 1));
-    c->hot_src = lights_d;
-    c->hot_n = params->num_lights;
     const LightCullParams& p = *params;
-    const uint64_t n = p.num_lights, nsup = tile_bin_supers(p);
+    hl_status s;
+    if ((s = ensure(c, c->hot, sizeof(HotLight) * (size_t)p.num_lights)) != HL_OK) return s;
     if (p.num_tiles_x == (p.screen_width + HL_TILE_SIZE - 1) / HL_TILE_SIZE &&
-        p.num_tiles_y == (p.screen_height + HL_TILE_SIZE - 1) / HL_TILE_SIZE && nsup * n <= 0xFFFFFFFFull) {
-        // the screen's tile grid: candidates binned per super-tile
-        if ((s = ensure(c, c->bits, 4 * cluster_bits_words((uint32_t)nsup, (uint32_t)n), true)) != HL_OK) return s;
-        if ((s = ensure(c, c->summary, 4 * cluster_summary_words((uint32_t)nsup, (uint32_t)n), true)) != HL_OK)
-            return s;
-        if ((s = ensure(c, c->raw, cluster_raw_bytes((uint32_t)nsup))) != HL_OK) return s;
-        const uint64_t tiles_n = (uint64_t)p.num_tiles_x * p.num_tiles_y;
-        if ((s = ensure(c, c->tilebin, 4 * (12 * tiles_n + 2 * nsup + nsup * n))) != HL_OK) return s;
-        float* planes = (float*)c->tilebin.p;
-        uint32_t* tb = (uint32_t*)(planes + 12 * tiles_n);
-        const TileBinScratch w{(uint32_t*)c->bits.p, (uint32_t*)c->summary.p, (uint32_t*)c->raw.p, tb, tb + nsup,
-                               tb + 2 * nsup, (uint32_t)(nsup * n), ctx_words(c) + 4, planes};
-        HL_HIP(c, launch_cull_tiles_binned(c->stream, camera_d, p, (const CullLight*)c->cull.p, lists_d, counts_d,
-                                           w));
+        p.num_tiles_y == (p.screen_height + HL_TILE_SIZE - 1) / HL_TILE_SIZE && p.num_tiles_x <= 0xFFFFu &&
+        p.num_tiles_y <= 0xFFFFu) {  // the screen's tile grid
+        if ((s = ensure(c, c->tilebin, tile_scratch_bytes(p.num_lights))) != HL_OK) return s;
+        HL_HIP(c, launch_cull_tiles_binned(c->stream, camera_d, p, lights_d, (HotLight*)c->hot.p, ctx_words(c) + 1,
+                                           c->tilebin.p, lists_d, counts_d));
     } else {
+        if ((s = ensure(c, c->cull, sizeof(CullLight) * (size_t)p.num_lights)) != HL_OK) return s;
+        HL_HIP(c, launch_prep(c->stream, lights_d, nullptr, p.num_lights, camera_d, (HotLight*)c->hot.p,
+                              (CullLight*)c->cull.p, ctx_words(c) + 1));
         HL_HIP(c, launch_cull_tiles(c->stream, camera_d, p, (const CullLight*)c->cull.p, lists_d, counts_d));
     }
+    c->hot_src = lights_d;
+    c->hot_n = p.num_lights;
     return HL_OK;
 }
 

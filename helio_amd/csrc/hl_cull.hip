@@ -1,8 +1,10 @@
 // hl_cull.hip -- light preparation and light assignment kernels for gfx950.
 //
 //  k_prep_lights      GpuLight[] -> HotLight[] (shading) + CullLight[] (culling)
-//  k_cull_tiles       reference 16-px tile lists (light_cull.wgsl:123-180), one
-//                     wavefront per tile, ballot + prefix-popcount compaction
+//  k_tile_prep/_cull  reference 16-px tile lists (light_cull.wgsl:123-180) of the
+//                     screen's grid, a super-tile per block
+//  k_cull_tiles       the same for any tile grid: one wavefront per tile, every
+//                     light tested, ballot + prefix-popcount compaction
 //  k_cluster_geom     per column: NDC rectangle and lateral planes; per cell:
 //                     the view-space AABB; its blocks past the cells prepare
 //                     the lights (as k_prep_lights) in the same launch
@@ -107,21 +109,24 @@ __global__ __launch_bounds__(256) void k_prep_zero(const GpuLight* __restrict__ 
 }
 
 // -------------------------------------------------------------- tile cull
-// The four planes of a 16x16 tile (light_cull.wgsl:123-150).
-__device__ __forceinline__ void tile_planes(const GpuCameraUniforms* __restrict__ cam, const LightCullParams& p,
-                                           uint32_t tile_x, uint32_t tile_y, float3 pl[4]) {
+// Plane k of a 16x16 tile: left, right, top, bottom (light_cull.wgsl:123-150).
+__device__ __forceinline__ float3 tile_plane(const GpuCameraUniforms* __restrict__ cam, const LightCullParams& p,
+                                             uint32_t tile_x, uint32_t tile_y, uint32_t k) {
 #pragma clang fp contract(off)
     const float fw = (float)p.screen_width, fh = (float)p.screen_height;
     const float ts = (float)HL_TILE_SIZE;
-    float ndc_left = ((float)tile_x * ts / fw) * 2.0f - 1.0f;
-    float ndc_right = fminf(((float)(tile_x + 1u) * ts / fw) * 2.0f - 1.0f, 1.0f);
-    float ndc_top = 1.0f - ((float)tile_y * ts / fh) * 2.0f;
-    float ndc_bottom = fmaxf(1.0f - ((float)(tile_y + 1u) * ts / fh) * 2.0f, -1.0f);
-    const float p00 = cam->proj[0], p11 = cam->proj[5];
-    pl[0] = hl_x_plane(p00, p11, ndc_left, ndc_bottom, ndc_left, ndc_top);
-    pl[1] = hl_x_plane(p00, p11, ndc_right, ndc_top, ndc_right, ndc_bottom);
-    pl[2] = hl_x_plane(p00, p11, ndc_left, ndc_top, ndc_right, ndc_top);
-    pl[3] = hl_x_plane(p00, p11, ndc_right, ndc_bottom, ndc_left, ndc_bottom);
+    const float l = ((float)tile_x * ts / fw) * 2.0f - 1.0f;
+    const float r = fminf(((float)(tile_x + 1u) * ts / fw) * 2.0f - 1.0f, 1.0f);
+    const float t = 1.0f - ((float)tile_y * ts / fh) * 2.0f;
+    const float b = fmaxf(1.0f - ((float)(tile_y + 1u) * ts / fh) * 2.0f, -1.0f);
+    // (l, b, l, t), (r, t, r, b), (l, t, r, t), (r, b, l, b)
+    return hl_x_plane(cam->proj[0], cam->proj[5], (k == 0u || k == 2u) ? l : r, (k == 0u || k == 3u) ? b : t,
+                      (k == 0u || k == 3u) ? l : r, (k == 0u || k == 2u) ? t : b);
+}
+__device__ __forceinline__ void tile_planes(const GpuCameraUniforms* __restrict__ cam, const LightCullParams& p,
+                                            uint32_t tile_x, uint32_t tile_y, float3 pl[4]) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) pl[k] = tile_plane(cam, p, tile_x, tile_y, k);
 }
 
 __device__ __forceinline__ bool tile_pass(const float3 pl[4], float4 c) {
@@ -1151,6 +1156,45 @@ __device__ __forceinline__ uint32_t list_bits(const uint32_t* words, uint32_t nw
     return total;
 }
 
+// Sets in words the bits of the lights j < nl whose column box holds the key's
+// column (boxes to a multiple of four) and that keep(j) accepts.  A lane takes
+// 4 kAhead lights at a time, their boxes loaded together, and sets the bits of
+// the few that pass; blocks start at different lights, so that they do not
+// all read the same lines at the same time.  Called by all NT threads; the
+// caller synchronises before the words are read.
+template <uint32_t NT, class F>
+__device__ __forceinline__ void scan_boxes(const uint32_t* __restrict__ boxes, uint32_t nl, uint32_t key,
+                                           uint32_t block, uint32_t* words, F&& keep) {
+    constexpr uint32_t kAhead = 8u;
+    const uint32_t t = threadIdx.x;
+    for (uint32_t w = t; w < (nl + 31u) / 32u; w += NT) words[w] = 0u;
+    __syncthreads();
+    const uint4* const cols = reinterpret_cast<const uint4*>(boxes);
+    const uint32_t quads = (nl + 3u) / 4u, groups = (quads + NT - 1u) / NT, rot = block % groups;
+    for (uint32_t g0 = 0; g0 < groups; g0 += kAhead) {
+        uint4 v[kAhead];
+#pragma unroll
+        for (uint32_t q = 0; q < kAhead; ++q) {
+            const uint32_t g = g0 + q + rot, j = (g < groups ? g : g - groups) * NT + t;
+            v[q] = make_uint4(kNoBox, kNoBox, kNoBox, kNoBox);
+            if (g0 + q < groups && j < quads) v[q] = cols[j];
+        }
+        uint32_t hits = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kAhead; ++q) {
+            hits |= box_has_column(v[q].x, key) ? 1u << (4u * q) : 0u;
+            hits |= box_has_column(v[q].y, key) ? 2u << (4u * q) : 0u;
+            hits |= box_has_column(v[q].z, key) ? 4u << (4u * q) : 0u;
+            hits |= box_has_column(v[q].w, key) ? 8u << (4u * q) : 0u;
+        }
+        for (; hits; hits &= hits - 1u) {
+            const uint32_t b = (uint32_t)__builtin_ctz(hits), g = g0 + (b >> 2) + rot;
+            const uint32_t j = 4u * ((g < groups ? g : g - groups) * NT + t) + (b & 3u);
+            if (keep(j)) atomicOr(&words[j >> 5], 1u << (j & 31u));
+        }
+    }
+}
+
 // The OR of a 64-bit word over the wave, in every lane (scalar).
 __device__ __forceinline__ uint64_t wave_or(uint64_t v) {
     const auto red = [](uint32_t x) {
@@ -1222,7 +1266,6 @@ __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const Colu
                                                 uint32_t nblocks, ColCountSmem<CHUNK>& sm, uint32_t* inline_slices) {
     constexpr uint32_t NT = kColThreads, kWaves = NT / 64u;
     static_assert(!INLINE || CHUNK == NT, "a light per thread");
-    constexpr uint32_t kAhead = 8u;  // loads of four lights' columns in flight per lane
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, n = a.num_lights;
     const ColBlock c = col_block(a, block, p.kb);
     float4 pr = make_float4(0.0f, 0.0f, 0.0f, 0.0f), dro = pr;
@@ -1265,37 +1308,9 @@ __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const Colu
             const uint64_t bal = hl_ballot(m);
             if (lane < 2u) sm.words[2u * wave + lane] = lane ? (uint32_t)(bal >> 32) : (uint32_t)bal;
         } else {
-            // a lane takes 4 kAhead lights at a time, their columns loaded
-            // together, and sets the bits of the few that hold its column;
-            // blocks start at different lights, so that they do not all read
-            // the same lines at the same time
-            for (uint32_t w = t; w < nw; w += NT) sm.words[w] = 0u;
-            __syncthreads();
-            const uint4* cols = reinterpret_cast<const uint4*>(p.box_col + l0);
-            const uint32_t quads = (nl + 3u) / 4u, groups = (quads + NT - 1u) / NT, rot = block % groups;
-            for (uint32_t g0 = 0; g0 < groups; g0 += kAhead) {
-                uint4 v[kAhead];
-#pragma unroll
-                for (uint32_t q = 0; q < kAhead; ++q) {
-                    const uint32_t g = g0 + q + rot, j = (g < groups ? g : g - groups) * NT + t;
-                    v[q] = make_uint4(kNoBox, kNoBox, kNoBox, kNoBox);
-                    if (g0 + q < groups && j < quads) v[q] = cols[j];
-                }
-                uint32_t hits = 0;
-#pragma unroll
-                for (uint32_t q = 0; q < kAhead; ++q) {
-                    hits |= box_has_column(v[q].x, key) ? 1u << (4u * q) : 0u;
-                    hits |= box_has_column(v[q].y, key) ? 2u << (4u * q) : 0u;
-                    hits |= box_has_column(v[q].z, key) ? 4u << (4u * q) : 0u;
-                    hits |= box_has_column(v[q].w, key) ? 8u << (4u * q) : 0u;
-                }
-                for (; hits && on; hits &= hits - 1u) {
-                    const uint32_t b = (uint32_t)__builtin_ctz(hits), g = g0 + (b >> 2) + rot;
-                    const uint32_t j = 4u * ((g < groups ? g : g - groups) * NT + t) + (b & 3u);
-                    if (part_column && !box_has_slices(p.box_slice[l0 + j], c.k0, k1)) continue;
-                    atomicOr(&sm.words[j >> 5], 1u << (j & 31u));
-                }
-            }
+            scan_boxes<NT>(p.box_col + l0, nl, key, block, sm.words, [&](uint32_t j) {
+                return on && (!part_column || box_has_slices(p.box_slice[l0 + j], c.k0, k1));
+            });
         }
         __syncthreads();
         const uint32_t total = list_bits<CHUNK / 32u, NT>(sm.words, nw, sm.list, sm.wave_sum);
@@ -1752,106 +1767,286 @@ __device__ __forceinline__ bool light_tiles(const GpuCameraUniforms* __restrict_
     return *tx1 >= *tx0 && *ty1 >= *ty0;
 }
 
-// One wavefront per light: the super-tiles its candidate tiles touch get
-// its bit (word-major bitmask over nsup cells, as the cluster cull's).
-// Block 0 also zeroes the scan tile sums that the count kernel adds to; the
-// blocks past the lights' (plane_blocks of them) build each tile's four
-// planes once, one thread per tile, for the list kernel's waves (a tile's
-// planes cost its wave some 800 VALU instructions of exact divisions and
-// square roots, the same in every lane).
-__global__ __launch_bounds__(256) void k_tile_bin(const GpuCameraUniforms* __restrict__ cam, LightCullParams p,
-                                                  const CullLight* __restrict__ cl, uint32_t* __restrict__ bits,
-                                                  uint32_t* __restrict__ summary,
-                                                  unsigned long long* __restrict__ tile_sums, uint32_t ntile_sums,
-                                                  float* __restrict__ planes, uint32_t plane_blocks) {
-    if (blockIdx.x < plane_blocks) {
-        const uint32_t tile = blockIdx.x * blockDim.x + threadIdx.x;
-        if (tile < p.num_tiles_x * p.num_tiles_y) {
-            float3 pl[4];
-            tile_planes(cam, p, tile % p.num_tiles_x, tile / p.num_tiles_x, pl);
-            float* o = planes + 12 * (size_t)tile;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                o[3 * k] = pl[k].x;
-                o[3 * k + 1] = pl[k].y;
-                o[3 * k + 2] = pl[k].z;
-            }
-        }
+// A block owns a super-tile of sx x sy tiles (at most 8 x 8; tile_plan): it
+// scans the lights' boxes in super-tiles as the column path does, lists the
+// candidates in LDS, finds the tiles of each one (a lane) as a bit per tile,
+// and a wave per row of tiles lists the candidates of each tile by ballot, the
+// first HL_MAX_LIGHTS_PER_TILE, in LDS; whole lists then go out in rows of
+// 256 bytes.  It stops when every tile is full.
+// A light in front of the camera is held against the columns and rows of the
+// super-tile first (tile_mask: the four plane tests are tests of a column or a
+// row but for rounding), and only against the planes of the tiles that this
+// leaves undecided; a tile's planes are built once, a plane per thread (some
+// 200 VALU instructions of exact divisions and square roots each).
+// k_tile_prep bounds the lights ahead of it, or every block all of them
+// (at most kColInline).
+// Measured (kernel times, us): 3840x2160 and 16384 lights 27 (prep 5, cull 22)
+// against 78 for the five launches over a bitmask of super-tiles and lights
+// that this replaces (prep 5.7, bin 15, count 15, fill 25, lists 17), 1280x720
+// and 64 lights 8.3 against 22.  What bounds it is latency, as in the column
+// path; half of the 4K launch is tile_mask.  Exact tests of every tile of the
+// rectangle in its place, with a store per list entry: 37 (and 8192 lights at
+// a time 30: two half-empty batches).
+constexpr uint32_t kTileMax = 64;  // tiles per block
+struct TileArgs {
+    const GpuCameraUniforms* cam;
+    const GpuLight* lights;
+    HotLight* hot;
+    uint32_t* feature_flags;
+    LightCullParams p;
+    uint32_t sx, sy, nsx;       // tiles per super-tile, super-tiles per row
+    uint32_t shift;             // boxes are in super-tiles >> shift (128 a side)
+    float4* vpos;               // per light (k_tile_prep): centre and range
+    uint2* rect;                // candidate tiles: x0 | y0 << 16, x1 | y1 << 16
+    uint32_t* box;              // the same in shifted super-tiles, as LightBox::col
+    uint32_t* lists;
+    uint32_t* counts;
+};
+
+// The candidate tiles of a light, and the super-tiles that hold them.
+__device__ __forceinline__ uint32_t tile_box(const TileArgs& a, float4 vpos, uint2* rect) {
+    int x0, x1, y0, y1;
+    *rect = make_uint2(1u, 0u);
+    if (!light_tiles(a.cam, a.p, vpos, &x0, &x1, &y0, &y1)) return kNoBox;
+    *rect = make_uint2((uint32_t)x0 | (uint32_t)y0 << 16, (uint32_t)x1 | (uint32_t)y1 << 16);
+    const uint32_t fx = a.sx << a.shift, fy = a.sy << a.shift;
+    return (uint32_t)x0 / fx | ((uint32_t)y0 / fy) << 8 | (127u - (uint32_t)x1 / fx) << 16 |
+           (127u - (uint32_t)y1 / fy) << 24;
+}
+
+__device__ __forceinline__ float4 light_vpos(float4 pr, uint32_t type, const float* __restrict__ v) {
+    return make_float4(hl_x_mat_row(v, 0, pr.x, pr.y, pr.z, 1.0f), hl_x_mat_row(v, 1, pr.x, pr.y, pr.z, 1.0f),
+                       hl_x_mat_row(v, 2, pr.x, pr.y, pr.z, 1.0f),
+                       type == HL_LIGHT_DIRECTIONAL ? __builtin_inff() : pr.w);
+}
+
+__global__ __launch_bounds__(64) void k_tile_prep(TileArgs a) {
+    const uint32_t i = blockIdx.x * 64u + threadIdx.x, n = a.p.num_lights;
+    if (i >= n) {
+        if (i < ((n + 3u) & ~3u)) a.box[i] = kNoBox;
         return;
     }
-    if (blockIdx.x == plane_blocks)
-        for (uint32_t i = threadIdx.x; i < ntile_sums; i += blockDim.x) tile_sums[i] = 0ull;
-    const uint32_t li = hl_uniform((blockIdx.x - plane_blocks) * 4u + (threadIdx.x >> 6));
-    if (li >= p.num_lights) return;
-    const float4 c = cl[li].vpos;
-    const float4 cu = make_float4(hl_uniform(c.x), hl_uniform(c.y), hl_uniform(c.z), hl_uniform(c.w));
-    int tx0, tx1, ty0, ty1;
-    if (!light_tiles(cam, p, cu, &tx0, &tx1, &ty0, &ty1)) return;
-    const uint32_t sx = (p.num_tiles_x + kSuperTile - 1u) / kSuperTile;
-    const uint32_t nsup = sx * ((p.num_tiles_y + kSuperTile - 1u) / kSuperTile);
-    const uint32_t s0x = (uint32_t)tx0 / kSuperTile, s1x = (uint32_t)tx1 / kSuperTile;
-    const uint32_t s0y = (uint32_t)ty0 / kSuperTile, s1y = (uint32_t)ty1 / kSuperTile;
-    const uint32_t nx = s1x - s0x + 1u, work = nx * (s1y - s0y + 1u);
-    const uint32_t word = li >> 5;
-    for (uint32_t t = threadIdx.x & 63u; t < work; t += 64u) {
-        const uint32_t iy = t / nx, ix = t - iy * nx;
-        const size_t sup = (size_t)(s0x + ix) + (size_t)sx * (s0y + iy);
-        __hip_atomic_fetch_or(hl_g(&bits[(size_t)word * nsup + sup]), 1u << (li & 31u), __ATOMIC_RELAXED,
-                              __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_or(hl_g(&summary[(size_t)(word >> 5) * nsup + sup]), 1u << (word & 31u),
-                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float4 v = light_vpos(*reinterpret_cast<const float4*>(a.lights[i].position_range), a.lights[i].light_type,
+                                a.cam->view);
+    uint2 rect;
+    a.vpos[i] = v;
+    a.box[i] = tile_box(a, v, &rect);
+    a.rect[i] = rect;
+    prep_one(a.lights, nullptr, n, a.cam, a.hot, nullptr, a.feature_flags, i);
+}
+
+// An edge of the super-tile's columns or rows in NDC, and the length
+// sqrt(1 + (edge / p)^2) of its plane's unnormalised normal.
+struct TileEdge {
+    float e, s;
+};
+template <uint32_t CHUNK>
+struct TileSmem {
+    alignas(16) float pl[kTileMax][12];  // the tiles' planes, tile y * 8 + x
+    TileEdge left[8], right[8], top[8], bottom[8];
+    uint32_t words[CHUNK / 32];
+    uint16_t list[CHUNK];
+    uint8_t tiles[kColBatch][8];         // a byte per row of tiles, a bit per tile
+    uint32_t out[kTileMax][HL_MAX_LIGHTS_PER_TILE];
+    uint32_t run[kTileMax];
+    uint32_t wave_sum[kColThreads / 64];
+    uint32_t open[2];                    // waves with a tile that still takes lights, per batch parity
+};
+
+// One axis of tile_mask: the tiles k in [k0, k1] that a centre at a = p c / zc
+// and a radius b = p r / zc certainly (sure) or possibly (may) pass: the lower
+// edge needs lo <= a + b s, the upper hi >= a - b s.
+template <class E>
+__device__ __forceinline__ void axis_mask(const E* lo, const E* hi, int k0, int k1, float a, float b, float margin,
+                                          uint32_t& sure, uint32_t& may) {
+    sure = may = 0u;
+    for (int k = k0; k <= k1; ++k) {
+        const float v = fminf(__builtin_fmaf(b, lo[k].s, a - lo[k].e), __builtin_fmaf(b, hi[k].s, hi[k].e - a));
+        const float m = margin + 1e-5f * (fabsf(a) + fabsf(b) * fmaxf(lo[k].s, hi[k].s) + 1.0f);
+        sure |= v > m ? 1u << k : 0u;
+        may |= !(v < -m) ? 1u << k : 0u;
     }
 }
 
-// One wavefront per tile: its super-tile's candidates (ascending) through
-// the exact plane test, the first HL_MAX_LIGHTS_PER_TILE kept in order.  The
-// candidates go through 256 at a time, four per lane (lane l takes the l-th
-// of each run of 64), their loads issued together.
-__global__ __launch_bounds__(256) void k_tile_lists(const float* __restrict__ planes, LightCullParams p,
-                                                    const CullLight* __restrict__ cl,
-                                                    const uint32_t* __restrict__ soff,
-                                                    const uint32_t* __restrict__ scnt,
-                                                    const uint32_t* __restrict__ spool,
-                                                    uint32_t* __restrict__ lists, uint32_t* __restrict__ counts) {
-    constexpr uint32_t kPer = 4;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6);
-    const uint32_t total = p.num_tiles_x * p.num_tiles_y;
-    if (tile >= total) return;
-    const uint32_t tile_x = tile % p.num_tiles_x, tile_y = tile / p.num_tiles_x;
-    const uint32_t sup = tile_x / kSuperTile + ((p.num_tiles_x + kSuperTile - 1u) / kSuperTile) * (tile_y / kSuperTile);
-    float3 pl[4];
+// The bytes of rows set in `rows`, each `cols`.
+__device__ __forceinline__ uint64_t mask_product(uint32_t rows, uint32_t cols) {
+    uint64_t m = 0;
+#pragma unroll
+    for (uint32_t y = 0; y < 8u; ++y) m |= (uint64_t)((rows >> y) & 1u ? cols : 0u) << (8u * y);
+    return m;
+}
+
+// The tiles of the super-tile that light c passes (bit y * 8 + x), of the
+// candidate rectangle [x0, x1] x [y0, y1].  In real numbers a light at view
+// distance zc > 0 passes a tile's left plane when l <= p00 (cx + r s) / zc
+// (s = sqrt(1 + l^2 / p00^2)), a condition of the tile's column alone, and so
+// on; the FP32 planes come from a cross product of two rays some theta
+// apart, whose components carry an error of at most about 1e-6: the plane
+// turns by 1e-6 / theta, moving the distance by that times |c|.  gx and gy
+// are four times that per |c| / zc, in NDC; what lies within takes the exact
+// test, and so does every tile for the other lights.
+template <uint32_t CHUNK>
+__device__ __forceinline__ uint64_t tile_mask(const TileSmem<CHUNK>& sm, float p00, float p11, float gx, float gy,
+                                              float4 c, int x0, int x1, int y0, int y1) {
+    if (x0 > x1 || y0 > y1) return 0ull;
+    uint32_t xs = 0u, xm = (2u << x1) - (1u << x0), ys = 0u, ym = (2u << y1) - (1u << y0);
+    const float zc = -c.z;
+    if (zc > 1e-4f && p00 > 0.0f && p11 > 0.0f && __builtin_isfinite(zc) && __builtin_isfinite(c.x) &&
+        __builtin_isfinite(c.y) && __builtin_isfinite(c.w)) {
+        const float iz = hl_f_rcp(zc), far = (fabsf(c.x) + fabsf(c.y) + zc) * iz;
+        axis_mask(sm.left, sm.right, x0, x1, p00 * c.x * iz, p00 * c.w * iz, gx * far, xs, xm);
+        // rows run downwards: the lower edge of the axis is the bottom
+        axis_mask(sm.bottom, sm.top, y0, y1, p11 * c.y * iz, p11 * c.w * iz, gy * far, ys, ym);
+    }
+    uint64_t in = mask_product(ys, xs);
+    for (uint64_t m = mask_product(ym, xm) & ~in; m; m &= m - 1ull) {
+        const uint32_t tile = (uint32_t)__builtin_ctzll(m);
+        const float4* q = reinterpret_cast<const float4*>(sm.pl[tile]);
+        const float4 q0 = q[0], q1 = q[1], q2 = q[2];
+        const float3 pl[4] = {make_float3(q0.x, q0.y, q0.z), make_float3(q0.w, q1.x, q1.y),
+                              make_float3(q1.z, q1.w, q2.x), make_float3(q2.y, q2.z, q2.w)};
+        if (tile_pass(pl, c)) in |= 1ull << tile;
+    }
+    return in;
+}
+
+template <uint32_t CHUNK, bool INLINE>
+__global__ __launch_bounds__(kColThreads) void k_tile_cull(TileArgs a) {
+    constexpr uint32_t NT = kColThreads;
+    static_assert(NT == 512, "a wave per row of tiles");
+    static_assert(kColBatch == NT, "a candidate per thread");
+    static_assert(!INLINE || CHUNK == NT, "a light per thread");
+    __shared__ TileSmem<CHUNK> sm;
+    float4* s_vpos = nullptr;
+    uint2* s_rect = nullptr;
+    if constexpr (INLINE) {
+        __shared__ float4 v[CHUNK];
+        __shared__ uint2 r[CHUNK];
+        s_vpos = v;
+        s_rect = r;
+    }
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = hl_uniform(t >> 6), n = a.p.num_lights;
+    const uint32_t sux = blockIdx.x % a.nsx, suy = blockIdx.x / a.nsx;
+    const uint32_t tx0 = sux * a.sx, ty0 = suy * a.sy;
+    const uint32_t nx = min(a.sx, a.p.num_tiles_x - tx0), ny = min(a.sy, a.p.num_tiles_y - ty0);
+    float4 pr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    uint32_t type = 0u;
+    if (INLINE && t < n) {  // in flight while the planes are built
+        pr = *reinterpret_cast<const float4*>(a.lights[t].position_range);
+        type = a.lights[t].light_type;
+    }
+    const float p00 = a.cam->proj[0], p11 = a.cam->proj[5];
+    float gx, gy;
     {
-        const float* q = planes + 12 * (size_t)tile;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            pl[k] = make_float3(hl_uniform(q[3 * k]), hl_uniform(q[3 * k + 1]), hl_uniform(q[3 * k + 2]));
-    }
-    const uint32_t n = hl_uniform(scnt[sup]);
-    const uint32_t* cand = spool + hl_uniform(soff[sup]);
-    uint32_t count = 0;
-    uint32_t* out = lists + (size_t)tile * HL_MAX_LIGHTS_PER_TILE;
-    for (uint32_t base = 0; base < n && count < HL_MAX_LIGHTS_PER_TILE; base += 64u * kPer) {
-        uint32_t idx[kPer];
-        float4 c[kPer];
-#pragma unroll
-        for (uint32_t q = 0; q < kPer; ++q) {
-            const uint32_t j = base + 64u * q + lane;
-            idx[q] = j < n ? cand[j] : 0xFFFFFFFFu;
+        const float fw = (float)a.p.screen_width, fh = (float)a.p.screen_height, ts = (float)HL_TILE_SIZE;
+        const uint32_t tile = t >> 2, x = tile & 7u, y = tile >> 3;
+        if (t < 4u * kTileMax && x < nx && y < ny) {
+            const float3 pl = tile_plane(a.cam, a.p, tx0 + x, ty0 + y, t & 3u);
+            float* o = &sm.pl[tile][3u * (t & 3u)];
+            o[0] = pl.x;
+            o[1] = pl.y;
+            o[2] = pl.z;
         }
+        if (t >= 256u && t < 256u + 32u) {  // the edges, as tile_plane's
+            const uint32_t k = t & 7u, side = (t >> 3) & 3u;
+            const bool row = side >= 2u;
+            const float at = (float)((row ? ty0 : tx0) + k + (side & 1u)) * ts / (row ? fh : fw) * 2.0f;
+            const float e = row ? fmaxf(1.0f - at, -1.0f) : fminf(at - 1.0f, 1.0f);
+            const float q = e * hl_f_rcp(row ? p11 : p00);
+            (side == 0u ? sm.left : side == 1u ? sm.right : side == 2u ? sm.top : sm.bottom)[k] =
+                TileEdge{e, __builtin_amdgcn_sqrtf(1.0f + q * q)};
+        }
+        // the smallest angles under which the block's tiles are seen: their
+        // NDC sizes (the screen's last tiles may be narrower), foreshortened
+        // at the screen's corners
+        const float ix = hl_f_rcp(p00), iy = hl_f_rcp(p11), corner = 1.0f + ix * ix + iy * iy;
+        const float wx = fminf((fw - (float)(tx0 + nx - 1u) * ts), ts) * 2.0f * hl_f_rcp(fw);
+        const float wy = fminf((fh - (float)(ty0 + ny - 1u) * ts), ts) * 2.0f * hl_f_rcp(fh);
+        gx = 4e-6f * p00 * corner * corner * hl_f_rcp(wy * iy);  // a column's planes span the tile's height
+        gy = 4e-6f * p11 * corner * corner * hl_f_rcp(wx * ix);
+    }
+    if (t < kTileMax) sm.run[t] = 0u;
+    if (t < 2u) sm.open[t] = 0u;
+    uint32_t batch = 0;
+    const uint32_t key = column_key(sux >> a.shift, suy >> a.shift);
+    bool open = true;  // some tile still takes lights (uniform)
+    for (uint32_t l0 = 0; l0 < n && open; l0 += CHUNK) {
+        const uint32_t nl = min(CHUNK, n - l0), nw = (nl + 31u) / 32u;
+        if (INLINE) {
+            bool m = false;
+            if (t < n) {
+                const float4 v = light_vpos(pr, type, a.cam->view);
+                uint2 rect;
+                m = box_has_column(tile_box(a, v, &rect), key);
+                s_vpos[t] = v;
+                s_rect[t] = rect;
+            }
+            const uint64_t bal = hl_ballot(m);
+            if (lane < 2u) sm.words[2u * wave + lane] = lane ? (uint32_t)(bal >> 32) : (uint32_t)bal;
+        } else {
+            if (l0) __syncthreads();  // the previous chunk's list is no longer read
+            scan_boxes<NT>(a.box + l0, nl, key, blockIdx.x, sm.words, [](uint32_t) { return true; });
+        }
+        __syncthreads();
+        const uint32_t total = list_bits<CHUNK / 32u, NT>(sm.words, nw, sm.list, sm.wave_sum);
+        for (uint32_t b0 = 0; b0 < total && open; b0 += kColBatch) {
+            uint64_t mask = 0;
+            if (b0 + t < total) {
+                const uint32_t li = sm.list[b0 + t];
+                const float4 c = INLINE ? s_vpos[li] : hl_ld4(a.vpos + l0 + li);
+                const uint2 r = INLINE ? s_rect[li] : a.rect[l0 + li];
+                // empty ranges where the boxes are coarser than the super-tiles
+                mask = tile_mask(sm, p00, p11, gx, gy, c, max((int)(r.x & 0xFFFFu) - (int)tx0, 0),
+                                 min((int)(r.y & 0xFFFFu) - (int)tx0, (int)nx - 1),
+                                 max((int)(r.x >> 16) - (int)ty0, 0), min((int)(r.y >> 16) - (int)ty0, (int)ny - 1));
+            }
+            *reinterpret_cast<uint64_t*>(sm.tiles[t]) = mask;
+            if (t == 0u) sm.open[(batch + 1u) & 1u] = 0u;  // read last before the previous barrier
+            __syncthreads();
+            // the wave's row of tiles
+            bool some = false;
+            if (wave < ny) {
+                uint32_t run[8];
 #pragma unroll
-        for (uint32_t q = 0; q < kPer; ++q)
-            c[q] = idx[q] != 0xFFFFFFFFu ? cl[idx[q]].vpos : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                for (uint32_t x = 0; x < 8u; ++x) run[x] = hl_uniform(sm.run[8u * wave + x]);
+                for (uint32_t g = 0; g < kColBatch && b0 + g < total; g += 64u) {
+                    const uint32_t row = sm.tiles[g + lane][wave];
+                    if (hl_ballot(row != 0u) == 0) continue;
+                    const uint32_t light = row ? l0 + sm.list[b0 + g + lane] : 0u;
 #pragma unroll
-        for (uint32_t q = 0; q < kPer; ++q) {
-            const bool pass = idx[q] != 0xFFFFFFFFu && tile_pass(pl, c[q]);
-            const uint64_t m = hl_ballot(pass);
-            const uint32_t pos = count + hl_prefix(m);
-            if (pass && pos < HL_MAX_LIGHTS_PER_TILE) out[pos] = idx[q];
-            count += (uint32_t)__popcll(m);
+                    for (uint32_t x = 0; x < 8u; ++x) {
+                        const bool in = (row >> x) & 1u;
+                        const uint64_t m = hl_ballot(in);
+                        const uint32_t pos = run[x] + hl_prefix(m);
+                        if (in && pos < HL_MAX_LIGHTS_PER_TILE) sm.out[8u * wave + x][pos] = light;
+                        run[x] += (uint32_t)__popcll(m);
+                    }
+                }
+#pragma unroll
+                for (uint32_t x = 0; x < 8u; ++x) {
+                    some = some || (x < nx && run[x] < HL_MAX_LIGHTS_PER_TILE);
+                    if (lane == x) sm.run[8u * wave + x] = run[x];
+                }
+            }
+            if (some && lane == 0u) atomicAdd(&sm.open[batch & 1u], 1u);
+            __syncthreads();  // and the masks and runs before the next batch's
+            open = sm.open[batch & 1u] != 0u;
+            ++batch;
         }
     }
-    if (lane == 0) counts[tile] = count < HL_MAX_LIGHTS_PER_TILE ? count : HL_MAX_LIGHTS_PER_TILE;
+    __syncthreads();
+    // a wave per row again: 64 entries of a tile at a time
+    for (uint32_t x = 0; x < nx && wave < ny; ++x) {
+        const uint32_t tile = (ty0 + wave) * a.p.num_tiles_x + tx0 + x;
+        const uint32_t cnt = min(sm.run[8u * wave + x], (uint32_t)HL_MAX_LIGHTS_PER_TILE);
+        static_assert(HL_MAX_LIGHTS_PER_TILE == 64, "an entry per lane");
+        if (lane < cnt) a.lists[(size_t)tile * HL_MAX_LIGHTS_PER_TILE + lane] = sm.out[8u * wave + x][lane];
+        if (lane == 0u) a.counts[tile] = cnt;
+    }
+    // the shading records, last: no wait stands on them
+    if (INLINE)
+        for (uint32_t i = blockIdx.x * NT + t; i < n; i += gridDim.x * NT)
+            prep_one(a.lights, nullptr, n, a.cam, a.hot, nullptr, a.feature_flags, i);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -1891,27 +2086,51 @@ hipError_t launch_cull_tiles(hipStream_t s, const GpuCameraUniforms* cam, const 
     return hipGetLastError();
 }
 
+// Tiles per super-tile: the smallest power of two that leaves at most
+// kTileBlocks blocks, all of them resident at once (two of 59 KB of LDS fit a
+// CU), at most kTileMax, at least as wide as high.  Twice as many blocks of half
+// the tiles, a quarter of them waiting for a place: 34 us at 4K and 16384
+// lights, 11.6 at 720p and 64.
+constexpr uint32_t kTileBlocks = 512;
+static void tile_plan(TileArgs& a) {
+    const uint64_t total = (uint64_t)a.p.num_tiles_x * a.p.num_tiles_y;
+    uint32_t log = 0;
+    while (log < 6u && total >> log > kTileBlocks) ++log;
+    a.sx = 1u << ((log + 1u) / 2u);
+    a.sy = 1u << (log / 2u);
+    a.nsx = (a.p.num_tiles_x + a.sx - 1u) / a.sx;
+    const uint32_t side = std::max(a.nsx, (a.p.num_tiles_y + a.sy - 1u) / a.sy);
+    a.shift = 0;
+    while ((side + (1u << a.shift) - 1u) >> a.shift > kColMaxSide) ++a.shift;
+}
+
+size_t tile_scratch_bytes(uint32_t num_lights) { return 28 * ((size_t)num_lights + 4); }
+
 hipError_t launch_cull_tiles_binned(hipStream_t s, const GpuCameraUniforms* cam, const LightCullParams& p,
-                                    const CullLight* cl, uint32_t* lists, uint32_t* counts,
-                                    const TileBinScratch& w) {
-    const uint32_t total = p.num_tiles_x * p.num_tiles_y;
-    if (total == 0) return hipSuccess;
-    const uint32_t nsup = tile_bin_supers(p);
-    const uint32_t W = (p.num_lights + 31u) / 32u, SW = (W + 31u) / 32u;
-    hipError_t e;
-    const uint32_t plane_blocks = (total + 255u) / 256u;
-    k_tile_bin<<<plane_blocks + (p.num_lights + 3) / 4, 256, 0, s>>>(
-        cam, p, cl, w.bits, w.summary, (unsigned long long*)((uint8_t*)w.raw + cluster_tile_sums_offset(nsup)),
-        cluster_scan_tiles(nsup), w.planes, plane_blocks);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    const uint32_t blocks = (nsup + 256u / kCellLanes - 1u) / (256u / kCellLanes);
-    k_cluster_count<<<blocks, 256, 0, s>>>(nsup, SW, w.bits, w.summary, w.raw, 0u);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    // the pool holds every (super-tile, light) pair: nothing is truncated
-    k_cluster_fill<<<blocks, 256, 0, s>>>(nsup, SW, w.raw, w.bits, w.summary, 0u, w.pool_cap, w.offsets,
-                                          w.counts, w.pool, w.flags, nullptr);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    k_tile_lists<<<(total + 3) / 4, 256, 0, s>>>(w.planes, p, cl, w.offsets, w.counts, w.pool, lists, counts);
+                                    const GpuLight* lights, HotLight* hot, uint32_t* feature_flags, void* scratch,
+                                    uint32_t* lists, uint32_t* counts) {
+    TileArgs a{};
+    a.cam = cam;
+    a.lights = lights;
+    a.hot = hot;
+    a.feature_flags = feature_flags;
+    a.p = p;
+    tile_plan(a);
+    const size_t n4 = ((size_t)p.num_lights + 3u) & ~(size_t)3u;
+    a.vpos = (float4*)scratch;
+    a.rect = (uint2*)(a.vpos + n4);
+    a.box = (uint32_t*)(a.rect + n4);
+    a.lists = lists;
+    a.counts = counts;
+    const uint32_t blocks = a.nsx * ((p.num_tiles_y + a.sy - 1u) / a.sy);
+    if (p.num_lights <= kColInline) {
+        k_tile_cull<kColInline, true><<<blocks, kColThreads, 0, s>>>(a);
+        return hipGetLastError();
+    }
+    k_tile_prep<<<(p.num_lights + 63u) / 64u, 64, 0, s>>>(a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_tile_cull<kColChunk, false><<<blocks, kColThreads, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -87,32 +87,15 @@ hipError_t launch_prep_zero(hipStream_t s, const GpuLight* lights, uint32_t n, c
 hipError_t launch_fill_u32(hipStream_t s, uint32_t* p, uint32_t v, size_t n);
 hipError_t launch_cull_tiles(hipStream_t s, const GpuCameraUniforms* cam, const LightCullParams& p,
                              const CullLight* cl, uint32_t* lists, uint32_t* counts);
-// The tile cull over candidates: each light's candidate tiles (a conservative
-// rectangle from necessary conditions of the plane test) are binned into
-// super-tiles of kSuperTile x kSuperTile tiles; the super-tiles' ascending
-// candidate lists come from the cluster count and fill kernels; each tile then
-// tests its super-tile's candidates in order with the exact plane test.  Same
-// lists as launch_cull_tiles when the tile grid is the screen's
-// (num_tiles = ceil(size / 16)).  bits and summary: as the cluster cull's
-// (zero before, zero after), over nsup = super-tiles cells.
-constexpr uint32_t kSuperTile = 4;
-struct TileBinScratch {
-    uint32_t* bits;     // nsup * ceil(L/32) words
-    uint32_t* summary;  // nsup * ceil(L/1024) words
-    uint32_t* raw;      // cluster_raw_bytes(nsup)
-    uint32_t* offsets;  // nsup
-    uint32_t* counts;   // nsup
-    uint32_t* pool;     // pool_cap
-    uint32_t pool_cap;  // nsup * L (no truncation)
-    uint32_t* flags;    // the fill's overflow word (never set: no cap, no truncation)
-    float* planes;      // 12 floats per tile: its four planes
-};
-inline uint32_t tile_bin_supers(const LightCullParams& p) {
-    return ((p.num_tiles_x + kSuperTile - 1u) / kSuperTile) * ((p.num_tiles_y + kSuperTile - 1u) / kSuperTile);
-}
+// The same lists when the tile grid is the screen's (num_tiles = ceil(size /
+// 16)): each light's candidate tiles (a conservative rectangle from necessary
+// conditions of the plane test), tested per super-tile of up to 64 tiles with
+// the exact plane test; builds the lights' shading records too (hot).
+// num_tiles below 65536 a side, num_lights > 0.
+size_t tile_scratch_bytes(uint32_t num_lights);
 hipError_t launch_cull_tiles_binned(hipStream_t s, const GpuCameraUniforms* cam, const LightCullParams& p,
-                                    const CullLight* cl, uint32_t* lists, uint32_t* counts,
-                                    const TileBinScratch& w);
+                                    const GpuLight* lights, HotLight* hot, uint32_t* feature_flags, void* scratch,
+                                    uint32_t* lists, uint32_t* counts);
 // Scratch of the clustered cull.  bits (ncell * ceil(L/32) words) and summary
 // (ncell * ceil(L/1024) words) must be zero before the first call; every call
 // leaves them zero again.
