@@ -213,8 +213,11 @@ enum ShadeMode : int {
     kModeExtended = 5,
     // flag on the forward-writing modes (forward, shadowed, extended): the
     // output target is RGBA16F (ShadeArgs::out_f16) instead of RGBA32F
-    kModeOutF16 = 8
+    kModeOutF16 = 8,
+    // flag on kModeForward: the view's wave tiles are shared (forward_split)
+    kModeShared = 16
 };
+constexpr int kModeMask = 7;
 // The fused forward + L2 adjoint shares a wave tile's lights among the block's
 // four waves on views of fewer than kFusedSplitBlocks block tiles: a 512^2
 // view has 1024 block tiles, 4096 waves of their own for 1024 SIMDs, and the
@@ -225,12 +228,32 @@ enum ShadeMode : int {
 constexpr uint32_t kFusedSplitBlocks = 4096;
 __host__ __device__ inline bool fused_split(uint32_t num_blocks) { return num_blocks < kFusedSplitBlocks; }
 
-// Work items of a shading launch over num_blocks block tiles: the backward
-// mode, and the fused mode when split, share each wave tile's lights among a
-// block's four waves, so their items are wave tiles (four per block tile).
-__host__ __device__ inline uint32_t shade_items(int mode, uint32_t num_blocks) {
-    return (mode == kModeBackward || (mode == kModeFusedL2 && fused_split(num_blocks))) ? 4u * num_blocks
-                                                                                       : num_blocks;
+// The forward mode shares a wave tile's lights among the block's four waves, by
+// the light's index modulo 4, on small views and on views that are small for
+// their lights: a 128^2 view has 256 wave tiles for 1024 SIMDs, and a wave that
+// walks a long list alone is one serial chain; on the other hand the four
+// waves repeat the tile's set-up and its walk.  Shading launch, us, unshared /
+// shared, by lights: 128^2 35 / 18 (256 lights), 117 / 40 (1024); 512^2 21 / 26
+// (64), 41 / 32 (256), 118 / 55 (1024); 1280x720 40 / 60 (256), 107 / 90 (1024),
+// 371 / 218 (4096); 1920x1080 52 / 113 (1024).  Hence up to 2^16 pixels, and up
+// to 2^20 with a light for every 1400.  The rule and the shares depend on the
+// view's size and lights only, so every path shading a view (single, batched,
+// any tile shape) adds the same sums.
+__host__ __device__ inline bool forward_split(uint32_t width, uint32_t height, uint32_t num_lights) {
+    const uint64_t px = (uint64_t)width * height;
+    return px <= (1u << 16) || (px <= (1u << 20) && px <= 1400ull * num_lights);
+}
+
+// Work items of a single-view shading launch of MODE (a ShadeMode with its
+// flags): the backward mode, the shared forward and the fused mode when split
+// share each wave tile's lights among a block's four waves, so their items are
+// wave tiles (four per block tile).  A batched launch shares under the fused
+// mode only.
+template <int MODE>
+__host__ __device__ inline uint32_t shade_items(const ShadeArgs& a) {
+    constexpr int M = MODE & kModeMask;
+    const bool split = M == kModeBackward || (MODE & kModeShared) || (M == kModeFusedL2 && fused_split(a.num_blocks));
+    return split ? 4u * a.num_blocks : a.num_blocks;
 }
 
 // Claim counters of one persistent shading launch: kShadeQueues counters,

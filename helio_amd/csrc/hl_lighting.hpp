@@ -4,6 +4,7 @@
 // arithmetic and exact decisions, and the wave-cooperative walk over a cell's
 // light list (lights refined against the wave's AABB and staged in LDS).
 #pragma once
+#include <type_traits>
 
 #include "hl_internal.hpp"
 
@@ -210,21 +211,28 @@ __device__ __forceinline__ bool eval_term(const HotLight& L, const Pixel& p, Ter
     t.Q = kPi * t.den * t.den + 0.0001f;
     t.el = t.ndl * (1.0f - p.kk) + p.kk1;
     t.den2 = 4.0f * p.ndv * t.ndl + 0.0001f;
-    float spec;
     if (kFull) {
         t.D = p.a2 * hl_f_rcp(t.Q);
         t.gl = t.ndl * hl_f_rcp(t.el);
         t.G = p.gv * t.gl;
-        spec = t.D * t.G * hl_f_rcp(t.den2);
+        const float spec = t.D * t.G * hl_f_rcp(t.den2);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            t.F[c] = p.f0[c] + (1.0f - p.f0[c]) * t.P;
+            t.B[c] = p.kd[c] + t.F[c] * (spec - p.kd[c]);  // (1 - F) kd + spec F
+        }
     } else {
         // D G / den2 with one reciprocal: a2 gv NdL / (Q el den2); for
-        // roughness in [0, 1] each factor lies in [1e-4, 4.1]
-        spec = p.a2gv * t.ndl * hl_f_rcp(t.Q * t.el * t.den2);
-    }
+        // roughness in [0, 1] each factor lies in [1e-4, 4.1].  The fused
+        // multiply-adds are written out: contraction depends on which block
+        // the compiler leaves an operation in, and kernels that divide the
+        // lights differently must round alike.
+        const float q = p.a2gv * t.ndl, r = hl_f_rcp(t.Q * t.el * t.den2);
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        t.F[c] = p.f0[c] + (1.0f - p.f0[c]) * t.P;
-        t.B[c] = p.kd[c] + t.F[c] * (spec - p.kd[c]);  // (1 - F) kd + spec F
+        for (int c = 0; c < 3; ++c) {
+            t.F[c] = __builtin_fmaf(1.0f - p.f0[c], t.P, p.f0[c]);
+            t.B[c] = __builtin_fmaf(t.F[c], __builtin_fmaf(q, r, -p.kd[c]), p.kd[c]);  // (1 - F) kd + spec F
+        }
     }
     return true;
 }
@@ -250,11 +258,28 @@ struct KeptState {
 // or with kept the next free one of the kept range), and the wave then visits
 // the set bits of the ballot (ascending lanes, i.e. list order) with uniform
 // reads of those slots.  a provides the grid (lists, counts, offsets,
-// lists_capacity) and the light records (lights, num_lights).
-template <int GRID, bool kKeep = false, class A, class F>
+// lists_capacity) and the light records (lights, num_lights).  share: a light
+// is taken only when (index & share.mask) == share.value.  OneClass: every
+// chunk's lights in list order; another classes object has the chunk's lights
+// visited class by class, the classes being the values of index & mask, and
+// calls next() after each (the sum of a class is then a plain running sum,
+// with nothing chosen per light).
+struct LightShare {
+    uint32_t mask = 0u, value = 0u;
+};
+struct OneClass {
+    static constexpr bool kOne = true;
+};
+template <class N>
+struct LightClasses {
+    static constexpr bool kOne = false;
+    uint32_t mask;  // 2^k - 1
+    N next;
+};
+template <int GRID, bool kKeep = false, class A, class F, class C = OneClass>
 __device__ __forceinline__ void walk_lights(const A& a, HotLight* s_l, const Pixel& p, bool valid,
                                             uint32_t cell, F&& f, KeptLights* kept = nullptr,
-                                            KeptState* ks = nullptr) {
+                                            KeptState* ks = nullptr, LightShare share = LightShare{}, C&& classes = C{}) {
     const uint32_t lane = hl_lane();
     uint64_t todo = hl_ballot(valid);
     while (todo) {
@@ -279,7 +304,7 @@ __device__ __forceinline__ void walk_lights(const A& a, HotLight* s_l, const Pix
             [[maybe_unused]] float4 q, l1, l2, l3, l4;  // kKeep: staged after the ballot
             if (j < cnt) {
                 idx = hl_g(list)[j];
-                if (idx < a.num_lights) {
+                if (idx < a.num_lights && (idx & share.mask) == share.value) {
                     // the whole record at once, so that staging it does not
                     // wait on a second load after the test
                     const HotLight* hp = a.lights + idx;
@@ -330,12 +355,26 @@ __device__ __forceinline__ void walk_lights(const A& a, HotLight* s_l, const Pix
                 }
             }
             hl_wave_sync();
-            uint32_t slot = first;
-            while (m) {
-                const uint32_t k = (uint32_t)__builtin_ctzll(m);
-                m &= m - 1u;
-                const HotLight L = s_l[keep ? slot++ : k];
-                f(L, hl_readlane(idx, k), mine);
+            if constexpr (!std::remove_reference_t<C>::kOne) {
+                if (m == 0u) continue;
+                for (uint32_t c = 0; c <= classes.mask; ++c) {
+                    uint64_t mc = m & hl_ballot((idx & classes.mask) == c);
+                    while (mc) {
+                        const uint32_t k = (uint32_t)__builtin_ctzll(mc);
+                        mc &= mc - 1u;
+                        const HotLight L = s_l[k];
+                        f(L, hl_readlane(idx, k), mine);
+                    }
+                    classes.next();
+                }
+            } else {
+                uint32_t slot = first;
+                while (m) {
+                    const uint32_t k = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1u;
+                    const HotLight L = s_l[keep ? slot++ : k];
+                    f(L, hl_readlane(idx, k), mine);
+                }
             }
             hl_wave_sync();
         }

@@ -124,12 +124,18 @@ struct ShadeSmem {
     HotLight light[4][kStage];
     ViewConst vc;
 };
+
 // LDS of the adjoint modes only (declared by their kernels alone, so that the
 // forward's occupancy is not charged for it)
 struct AdjSmem {
     KeptLights kept[4];      // fused: the lights each wave's walk visited
     float gl[4][3][64];      // fused: the waves' partial radiance sums
     float red[1][4][5][64];  // the waves' partial per-pixel gradient sums
+};
+
+// LDS of the batched forward alone: the waiting class sums of each wave
+struct ClassSmem {
+    float sum[4][9][64];
 };
 
 // Fills sm.vc from the view's arguments; the caller synchronises the block
@@ -318,9 +324,18 @@ __device__ __forceinline__ void adjoint_light(const ShadeArgs& a, const HotLight
     }
 }
 
+// How the forward mode divides a view that forward_split holds for.  kOwn: the
+// view is not one; a wave has its own tile and one sum.  kShare: the block's
+// four waves share a tile, each the lights of one index modulo 4.  kClasses
+// (batched launches, which have waves enough and cannot choose per view at
+// compile time): a wave has its own tile and keeps the four sums apart on
+// such a view, so that the pixel is kShare's bit for bit.
+enum LightDivision : int { kOwn = 0, kShare = 1, kClasses = 2 };
+
 // Every mode but the fused forward + adjoint (fused_tile).
-template <int FA, int FN, int GRID, int MODE, bool F16 = false>
-__device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, ShadeSmem& sm, AdjSmem* as) {
+template <int FA, int FN, int GRID, int MODE, bool F16 = false, int DIV = kOwn>
+__device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, ShadeSmem& sm, AdjSmem* as,
+                                           ClassSmem* cl = nullptr) {
     static_assert(MODE != kModeFusedL2, "fused_tile");
     const ViewConst& vc = sm.vc;
     b = hl_uniform(b);  // the item is the block's: its tile arithmetic stays scalar
@@ -329,22 +344,26 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     // The backward mode splits a wave tile's adjoint over the block's four
     // waves (every fourth light each; the items are wave tiles, four per block
     // tile): its per-light work is several times the forward's, and the
-    // heaviest tiles would otherwise set the launch's length.  The other modes
-    // give each wave its own tile of the block tile.
-    constexpr bool kSplit = kAdj;
+    // heaviest tiles would otherwise set the launch's length.  The forward
+    // mode shares a wave tile's lights alike under kShare; else each wave has
+    // its own tile of the block tile.
+    constexpr bool kRC = MODE == kModeExtended;
+    constexpr bool kExt = MODE == kModeShadowed || kRC;  // exact N, shadow_factor
+    constexpr bool kFwd = MODE == kModeForward || kExt;
+    constexpr bool kShared = MODE == kModeForward && DIV == kShare;
+    constexpr bool split = kAdj || kShared;
+    [[maybe_unused]] const bool classes =
+        MODE == kModeForward && DIV == kClasses && forward_split(a.width, a.height, a.num_lights);
     const uint32_t twl = a.tw_log2, tw = 1u << twl;
     const uint32_t th = 64u >> twl;
-    const uint32_t bt = kSplit ? b >> 2 : b, sub = kSplit ? (b & 3u) : wave;
+    const uint32_t bt = split ? b >> 2 : b, sub = split ? (b & 3u) : wave;
     const uint32_t bx = bt % a.block_tiles_x, by = bt / a.block_tiles_x;
     const uint32_t x = bx * (4u * tw) + sub * tw + (lane & (tw - 1u));
     const uint32_t y = by * th + (lane >> twl);
     const bool inside = x < a.width && y < a.height;
     const float depth = inside ? hl_load_depth(a.depth, x, y) : 1.0f;
     const bool valid = inside && depth < 1.0f;
-    const bool lead = !kSplit || wave == 0u;  // writes the tile's shared results
-    constexpr bool kRC = MODE == kModeExtended;
-    constexpr bool kExt = MODE == kModeShadowed || kRC;  // exact N, shadow_factor
-    constexpr bool kFwd = MODE == kModeForward || kExt;
+    const bool lead = !split || wave == 0u;  // writes the tile's shared results
     constexpr bool kWrites = kFwd;
     // the pixel's address, computed once (8 B per pixel for RGBA16F, else 16)
     constexpr bool out_f16 = F16;
@@ -369,7 +388,7 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
 
     // ---- debug views (deferred_lighting.wgsl:1032-1038)
     if (kFwd && a.debug_mode != 0u) {
-        if (valid) {
+        if (valid && lead) {
             float4 o;
             if (a.debug_mode == 5u)
                 o = make_float4(p.nx * 0.5f + 0.5f, p.ny * 0.5f + 0.5f, p.nz * 0.5f + 0.5f, 1.0f);
@@ -427,8 +446,20 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
             amb[c] = (hemi * (1.0f - w) + diff * w) * p.ao + (c == 0 ? E.x : (c == 1 ? E.y : E.z));
         }
     }
+    // kClasses: the sums of the other three classes of lights wait in LDS (each
+    // lane its own words), the next one at `head`: held in registers they cost
+    // 9 spills under the kernel's 5 waves per SIMD
+    [[maybe_unused]] uint32_t head = 0u;
+    [[maybe_unused]] float(*sums)[64] = nullptr;
+    if constexpr (DIV == kClasses) {
+        sums = cl->sum[wave];
+        if (classes) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k) sums[k][lane] = 0.0f;
+        }
+    }
     if (MODE != kModeBackward) {
-        walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t, bool mine) {
+        const auto term = [&](const HotLight& L, uint32_t, bool mine) {
             if (!mine) return;
             Term t;
             if (eval_term<false>(L, p, t)) {
@@ -442,11 +473,46 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
                         aw *= shadow_factor(a.shadow, L, w >> 28, w & 0x0FFFFFFFu, p.wx, p.wy, p.wz, p.nx, p.ny,
                                             p.nz, (float)x + 0.5f, (float)y + 0.5f, vc.eye);
                 }
-                lo[0] += t.B[0] * (L.p1.x * aw);
-                lo[1] += t.B[1] * (L.p1.y * aw);
-                lo[2] += t.B[2] * (L.p1.z * aw);
+                lo[0] = __builtin_fmaf(t.B[0], L.p1.x * aw, lo[0]);
+                lo[1] = __builtin_fmaf(t.B[1], L.p1.y * aw, lo[1]);
+                lo[2] = __builtin_fmaf(t.B[2], L.p1.z * aw, lo[2]);
             }
-        });
+        };
+        if constexpr (DIV == kClasses) {
+            const auto rotate = [&] {
+                if (!classes) return;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const float first = lo[c];
+                    lo[c] = sums[3u * head + c][lane];
+                    sums[3u * head + c][lane] = first;
+                }
+                head = head == 2u ? 0u : head + 1u;
+            };
+            walk_lights<GRID>(a, s_l, p, valid, cell, term, nullptr, nullptr, LightShare{},
+                              LightClasses<decltype(rotate)>{classes ? 3u : 0u, rotate});
+        } else {
+            walk_lights<GRID>(a, s_l, p, valid, cell, term, nullptr, nullptr,
+                              kShared ? LightShare{3u, wave} : LightShare{});
+        }
+    }
+    if (DIV == kClasses && classes) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            for (uint32_t k = 0; k < 3u; ++k) lo[c] += sums[3u * ((head + k) % 3u) + c][lane];
+        }
+    }
+    if (kShared) {  // the partial sums, in the waves' staging space, added in wave order by the first wave
+        const auto part = [&](uint32_t w) { return reinterpret_cast<float*>(sm.light[w]); };
+        if (!lead) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) part(wave)[64 * c + lane] = lo[c];
+        }
+        __syncthreads();  // the block's: all its waves are on this tile
+        if (!lead) return;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            lo[c] = ((lo[c] + part(1)[64 * c + lane]) + part(2)[64 * c + lane]) + part(3)[64 * c + lane];
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) o[c] = lo[c] + amb[c];
@@ -784,11 +850,12 @@ constexpr int shade_min_blocks() {
                : (MODE == kModeForward || MODE == kModeShadowed || MODE == kModeExtended ? 4 : 1);
 }
 
-// MODE: a ShadeMode, with kModeOutF16 set for an RGBA16F target
+// MODE: a ShadeMode, with kModeOutF16 set for an RGBA16F target and kModeShared
+// for a forward view whose wave tiles are shared (forward_split)
 template <int FA, int FN, int GRID, int MODE>
-__global__ __launch_bounds__(256, (shade_min_blocks<(MODE & ~kModeOutF16), FA>())) void k_shade(
+__global__ __launch_bounds__(256, (shade_min_blocks<(MODE & kModeMask), FA>())) void k_shade(
     ShadeArgs a, uint32_t* __restrict__ queue, uint32_t* __restrict__ queue_next) {
-    constexpr int M = MODE & ~kModeOutF16;
+    constexpr int M = MODE & kModeMask;
     __shared__ ShadeSmem sm;
     __shared__ ClaimSmem cs;
     AdjSmem* as = nullptr;
@@ -798,9 +865,9 @@ __global__ __launch_bounds__(256, (shade_min_blocks<(MODE & ~kModeOutF16), FA>()
     }
     if (blockIdx.x == 0 && threadIdx.x < kShadeQueues) queue_next[threadIdx.x * kShadeQueueStride] = 0u;
     load_view_const(a, sm);  // published by the first claim's barrier
-    claim_items(shade_items(M, a.num_blocks), queue, cs, [&](uint32_t t) {
+    claim_items(shade_items<MODE>(a), queue, cs, [&](uint32_t t) {
         if constexpr (M == kModeFusedL2) fused_tile<FA, FN, GRID>(a, t, sm, *as);
-        else shade_tile<FA, FN, GRID, M, (MODE & kModeOutF16) != 0>(a, t, sm, as);
+        else shade_tile<FA, FN, GRID, M, (MODE & kModeOutF16) != 0, (MODE & kModeShared) ? kShare : kOwn>(a, t, sm, as);
     });
 }
 
@@ -834,12 +901,17 @@ __global__ __launch_bounds__(256, MODE == kModeForward ? 5 : 1) void k_shade_bat
         __shared__ AdjSmem adj;
         as = &adj;
     }
+    ClassSmem* cl = nullptr;
+    if constexpr (MODE == kModeForward) {
+        __shared__ ClassSmem classes;
+        cl = &classes;
+    }
     uint32_t first = 1u, end = 0u, v = 0u;  // item range of the staged view (none yet), its index
     if (nspans == 1u) {
         load_view_const(one, sm);  // published by the first claim's barrier
         claim_items(num_items, queue, cs, [&](uint32_t it) {
             if constexpr (MODE == kModeFusedL2) fused_tile<FA, FN, HL_GRID_CLUSTERS>(one, it, sm, *as);
-            else shade_tile<FA, FN, HL_GRID_CLUSTERS, MODE>(one, it, sm, as);
+            else shade_tile<FA, FN, HL_GRID_CLUSTERS, MODE, false, kClasses>(one, it, sm, as, cl);
         });
     } else claim_items(num_items, queue, cs, [&](uint32_t it) {
         it = hl_uniform(it);  // block-uniform: every thread read the same claim
@@ -861,7 +933,7 @@ __global__ __launch_bounds__(256, MODE == kModeForward ? 5 : 1) void k_shade_bat
         // to be uniform
         const ShadeArgs& ra = *(const ShadeArgs*)&views[hl_uniform(v)].sa;
         if constexpr (MODE == kModeFusedL2) fused_tile<FA, FN, HL_GRID_CLUSTERS>(ra, it - first, sm, *as);
-        else shade_tile<FA, FN, HL_GRID_CLUSTERS, MODE>(ra, it - first, sm, as);
+        else shade_tile<FA, FN, HL_GRID_CLUSTERS, MODE, false, kClasses>(ra, it - first, sm, as, cl);
     });
     // The last block out clears the claim counters for the next launch, so a
     // captured graph replays this launch unchanged.  Blocks that have finished
@@ -963,12 +1035,12 @@ template <int FA, int FN, int MODE>
 static hipError_t launch_grid(hipStream_t s, const ShadeArgs& a, uint32_t* queue, uint32_t* queue_next) {
     if (a.grid_mode == HL_GRID_TILES)
         k_shade<FA, FN, HL_GRID_TILES, MODE>
-            <<<persistent_blocks<FA, FN, HL_GRID_TILES, MODE>(shade_items(MODE & ~kModeOutF16, a.num_blocks)), 256,
+            <<<persistent_blocks<FA, FN, HL_GRID_TILES, MODE>(shade_items<MODE>(a)), 256,
                0, s>>>(
                 a, queue, queue_next);
     else
         k_shade<FA, FN, HL_GRID_CLUSTERS, MODE>
-            <<<persistent_blocks<FA, FN, HL_GRID_CLUSTERS, MODE>(shade_items(MODE & ~kModeOutF16, a.num_blocks)),
+            <<<persistent_blocks<FA, FN, HL_GRID_CLUSTERS, MODE>(shade_items<MODE>(a)),
                256, 0, s>>>(
                 a, queue, queue_next);
     return hipGetLastError();
@@ -986,6 +1058,9 @@ static hipError_t launch_fmt(hipStream_t s, int set, const ShadeArgs& a, uint32_
 hipError_t launch_shade(hipStream_t s, int gbuf_set, int mode, const ShadeArgs& a, uint32_t* queue,
                         uint32_t* queue_next) {
     if (a.num_blocks == 0) return hipSuccess;
+    if (mode == kModeForward && forward_split(a.width, a.height, a.num_lights))
+        return a.out_f16 ? launch_fmt<kModeForward | kModeShared | kModeOutF16>(s, gbuf_set, a, queue, queue_next)
+                         : launch_fmt<kModeForward | kModeShared>(s, gbuf_set, a, queue, queue_next);
     if (a.out_f16) {  // the modes that write the radiance alone take an RGBA16F target
         switch (mode) {
             case kModeForward: return launch_fmt<kModeForward | kModeOutF16>(s, gbuf_set, a, queue, queue_next);
