@@ -616,6 +616,24 @@ __device__ __forceinline__ float dpp_sum(float v) {
     return hl_readlane(v, 63);
 }
 
+// Four sums over the wave at once: lane l returns the sum of v(l % 4).  The
+// first two steps halve the values with the lanes (each lane keeps one of a
+// pair and adds its neighbour's copy), so the rest is one reduction: 17 VALU
+// instructions against 24 and a selection for four dpp_sum.
+__device__ __forceinline__ float dpp_sum4(float v0, float v1, float v2, float v3) {
+    const uint32_t lane = hl_lane();
+    const bool odd = (lane & 1u) != 0u, high = (lane & 2u) != 0u;
+    const float a = (odd ? v1 : v0) + hl_dpp<0xB1>(0.0f, odd ? v0 : v1);  // quad_perm [1,0,3,2]
+    const float b = (odd ? v3 : v2) + hl_dpp<0xB1>(0.0f, odd ? v2 : v3);
+    float e = (high ? b : a) + hl_dpp<0x4E>(0.0f, high ? a : b);          // quad_perm [2,3,0,1]
+    e = e + hl_dpp<0x124>(0.0f, e);                                       // row_ror:4
+    e = e + hl_dpp<0x128>(0.0f, e);                                       // row_ror:8
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(e), __float_as_uint(e), false, false);
+    e = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(e), __float_as_uint(e), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+}
+
 // Placed in a rarely taken block, keeps the optimizer from executing the block
 // unconditionally and selecting its result (an empty volatile asm statement
 // has side effects, so the block cannot be speculated).

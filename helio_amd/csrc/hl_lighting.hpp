@@ -29,14 +29,17 @@ struct Pixel {
 };
 
 // Per-(pixel, light) quantities of pbr_direct_light (deferred_lighting.wgsl:699-820).
+// The last two rows are the adjoint's (kFull): spec = D G / den2 = q1 NdL =
+// a2 w0 NdL, and dB/dF = spec - kd.
 struct Term {
     float lx, ly, lz;
-    float rad[3];
     float ndl;
     float d, inv_d, att0, fall, s, dsdcos, atten;
     float hx, hy, hz, inv_h;
-    float hdv, u, P, ndh, a2, den, Q, D, el, gl, G, den2;
+    float hdv, u, P, ndh, den, Q, el, den2;
     float F[3], B[3];
+    float inv_q, inv_el, inv_den2;
+    float w0, q1, spec, dB[3];
 };
 
 // Range test of deferred_lighting.wgsl:1128-1131 (dist > range rejects)
@@ -180,11 +183,6 @@ __device__ __forceinline__ bool eval_term(const HotLight& L, const Pixel& p, Ter
     t.s = s;
     t.dsdcos = dsdcos;
     t.atten = atten;
-    if (kFull) {
-        t.rad[0] = L.p1.x * atten;
-        t.rad[1] = L.p1.y * atten;
-        t.rad[2] = L.p1.z * atten;
-    }
     t.ndl = fmaxf(p.nx * t.lx + p.ny * t.ly + p.nz * t.lz, 0.0f);
     if (t.ndl == 0.0f) return false;
     // H = normalize(V + L) and N.H in the shader's order: for smooth surfaces
@@ -207,19 +205,21 @@ __device__ __forceinline__ bool eval_term(const HotLight& L, const Pixel& p, Ter
     t.u = fminf(fmaxf(1.0f - t.hdv, 0.0f), 1.0f);
     const float u2 = t.u * t.u;
     t.P = u2 * u2 * t.u;
-    t.a2 = p.a2;
     t.Q = kPi * t.den * t.den + 0.0001f;
     t.el = t.ndl * (1.0f - p.kk) + p.kk1;
     t.den2 = 4.0f * p.ndv * t.ndl + 0.0001f;
     if (kFull) {
-        t.D = p.a2 * hl_f_rcp(t.Q);
-        t.gl = t.ndl * hl_f_rcp(t.el);
-        t.G = p.gv * t.gl;
-        const float spec = t.D * t.G * hl_f_rcp(t.den2);
+        t.inv_q = hl_f_rcp(t.Q);
+        t.inv_el = hl_f_rcp(t.el);
+        t.inv_den2 = hl_f_rcp(t.den2);
+        t.w0 = p.gv * t.inv_el * (t.inv_q * t.inv_den2);
+        t.q1 = p.a2 * t.w0;
+        t.spec = t.q1 * t.ndl;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            t.F[c] = p.f0[c] + (1.0f - p.f0[c]) * t.P;
-            t.B[c] = p.kd[c] + t.F[c] * (spec - p.kd[c]);  // (1 - F) kd + spec F
+            t.F[c] = __builtin_fmaf(1.0f - p.f0[c], t.P, p.f0[c]);
+            t.dB[c] = t.spec - p.kd[c];
+            t.B[c] = __builtin_fmaf(t.F[c], t.dB[c], p.kd[c]);  // (1 - F) kd + spec F
         }
     } else {
         // D G / den2 with one reciprocal: a2 gv NdL / (Q el den2); for

@@ -20,92 +20,89 @@
 
 namespace hl {
 
-// Reverse-mode derivative of one active term given dL/dout (gl).  Per-pixel
-// gradients accumulate into dA (albedo), dR (roughness), dM (metallic); the
-// light's position and intensity gradients are returned in g (x, y, z, I).
-__device__ __forceinline__ void adjoint_term(const HotLight& L, const Pixel& p, const Term& t,
-                                             const float gl[3], float dA[3], float& dR, float& dM,
-                                             float4& g) {
-    const float m = p.metal, r = p.rough;
-    const float inv_den2 = hl_f_rcp(t.den2);
-    const float DG_den2 = t.D * t.G * inv_den2;
-    const float invQ = hl_f_rcp(t.Q);
-    // dD/dr and dG/dr (pbr_eval.wgsl:12-43)
-    const float dDdr = (invQ - t.a2 * 2.0f * kPi * t.den * t.ndh * t.ndh * invQ * invQ) * 4.0f * r * r * r;
-    const float inv_ev = hl_f_rcp(p.ev), inv_el = hl_f_rcp(t.el);
-    const float dgdk_v = -p.ndv * (1.0f - p.ndv) * inv_ev * inv_ev;
-    const float dgdk_l = -t.ndl * (1.0f - t.ndl) * inv_el * inv_el;
-    const float dGdr = (dgdk_v * t.gl + p.gv * dgdk_l) * (r + 1.0f) * 0.25f;
-    const float dSdr = (dDdr * t.G + t.D * dGdr) * inv_den2;
-    const float atten = t.att0 * t.fall * t.s;
-    float adj_NdL = 0.0f, adj_atten = 0.0f, adj_D = 0.0f, adj_G = 0.0f, adj_den2 = 0.0f, adj_P = 0.0f;
-    float dI = 0.0f;
-    // color = (color * intensity) / intensity: an active term has radiance
-    // >= 0.002, hence intensity != 0
-    const float inv_I = hl_f_rcp(L.p3.y);
-    const float cI[3] = {L.p1.x, L.p1.y, L.p1.z};
+// What a pixel's material gradients need of its lights.  With gw = dL/dout x
+// radiance x NdL per channel, 1 - F = (1 - f0)(1 - P) and k, F0 and the
+// roughness powers constant over the lights, the gradients are linear in
+//   h = sum gw (1 - P)     y = sum gw (1 - P) (spec - kd)   (per channel)
+//   r1: the derivative of D by its a2 = r^4     r2: of G by its k,
+// so the loop adds eight sums and the per-pixel factors go on at the end
+// (adjoint_pixel).
+struct MaterialSums {
+    float h[3] = {0.0f, 0.0f, 0.0f}, y[3] = {0.0f, 0.0f, 0.0f}, r1 = 0.0f, r2 = 0.0f;
+};
+
+// dA (albedo), dR (roughness), dM (metallic) of the pixel from its sums.
+__device__ __forceinline__ void adjoint_pixel(const Pixel& p, const MaterialSums& s, float dA[3], float& dR,
+                                              float& dM) {
+    dM = 0.0f;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        const float W = t.rad[c] * t.ndl;
-        const float gw = gl[c] * W;
-        const float dBdF = -(1.0f - m) * p.alb[c] * kInvPi + DG_den2;
-        const float kD = (1.0f - t.F[c]) * p.one_m;
-        dA[c] += gw * (kD * kInvPi + (p.f0_free[c] ? m * (1.0f - t.P) * dBdF : 0.0f));
-        dM += gw * (-(1.0f - t.F[c]) * p.alb[c] * kInvPi +
-                    (p.f0_free[c] ? (p.alb[c] - 0.04f) * (1.0f - t.P) * dBdF : 0.0f));
-        dR += gw * dSdr * t.F[c];
-        dI += gl[c] * t.B[c] * cI[c] * inv_I * atten * t.ndl;
-        const float adj_B = gw;
-        adj_NdL += gl[c] * t.B[c] * t.rad[c];
-        adj_atten += gl[c] * t.B[c] * t.ndl * cI[c];
-        adj_D += adj_B * t.G * t.F[c] * inv_den2;
-        adj_G += adj_B * t.D * t.F[c] * inv_den2;
-        adj_den2 -= adj_B * DG_den2 * t.F[c] * inv_den2;
-        adj_P += adj_B * dBdF * (1.0f - p.f0[c]);
+        const float x = (1.0f - p.f0[c]) * s.h[c];  // sum gw (1 - F)
+        dA[c] = p.one_m * kInvPi * x + (p.f0_free[c] ? p.metal * s.y[c] : 0.0f);
+        dM += -kInvPi * p.alb[c] * x + (p.f0_free[c] ? (p.alb[c] - 0.04f) * s.y[c] : 0.0f);
     }
-    g = make_float4(0.0f, 0.0f, 0.0f, dI);
+    dR = 4.0f * p.rough * p.rough * p.rough * s.r1 - (p.rough + 1.0f) * 0.25f * s.r2;
+}
+
+// Reverse-mode derivative of one active term given dL/dout (gl): the material
+// sums, and in g the light's gradients by position (x, y, z) and by intensity
+// times the intensity (w).  cv = (1 - NdV) / ev.
+// Every partial of spec = D G / den2 is spec times a logarithmic derivative
+// (pbr_eval.wgsl:12-43), and the three channels enter through three dot
+// products (with F, with dB/dF (1 - F0), with the light's colour).  Against
+// channel-by-channel adjoints of D, G and den2 and four separate wave sums:
+// 773x431 backward 85 -> 71 us, 512^2 fused 70 -> 63 us, two 1032x1104 eyes
+// fused 280 -> 255 us; held to 128 VGPRs (4 waves per SIMD, 7 to 40 spills) no
+// faster, 512^2 80 us.
+__device__ __forceinline__ void adjoint_term(const HotLight& L, const Pixel& p, const Term& t,
+                                             const float gl[3], float cv, MaterialSums& m, float4& g) {
+    const float aw = t.atten * t.ndl;
+    const float one_P = 1.0f - t.P;
+    const float col[3] = {L.p1.x, L.p1.y, L.p1.z};
+    float S = 0.0f, GF = 0.0f, adj_P = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const float gc = gl[c] * col[c];
+        const float gw = gc * aw;
+        const float e = gw * t.dB[c];
+        S += gc * t.B[c];
+        GF += gw * t.F[c];
+        adj_P += e * (1.0f - p.f0[c]);
+        m.h[c] += gw * one_P;
+        m.y[c] += e * one_P;
+    }
+    const float E = GF * t.spec;
+    const float pn = (2.0f * kPi) * t.den * t.inv_q * t.ndh;  // dlnD/dNdH = 2 (1 - a2) pn
+    m.r1 += GF * (t.w0 * t.ndl) * (1.0f - p.a2 * pn * t.ndh);
+    m.r2 += E * (cv + (1.0f - t.ndl) * t.inv_el);
+    g = make_float4(0.0f, 0.0f, 0.0f, S * aw);
     if (__builtin_isinf(L.p0.w)) return;  // directional: no position
-    float ahx = 0.0f, ahy = 0.0f, ahz = 0.0f;
-    if (t.hdv > 0.0f && t.u > 0.0f) {
-        const float u2 = t.u * t.u;
-        const float a = adj_P * (-5.0f * u2 * u2);
-        ahx += a * p.vx;
-        ahy += a * p.vy;
-        ahz += a * p.vz;
-    }
-    if (t.ndh > 0.0f) {
-        const float dDdNdH = -t.a2 * invQ * invQ * (2.0f * kPi * t.den) * (2.0f * t.ndh * (t.a2 - 1.0f));
-        const float a = adj_D * dDdNdH;
-        ahx += a * p.nx;
-        ahy += a * p.ny;
-        ahz += a * p.nz;
-    }
-    adj_NdL += adj_G * p.gv * (p.kk + 0.0001f) * inv_el * inv_el;
-    adj_NdL += adj_den2 * 4.0f * p.ndv;
-    const float hd = t.hx * ahx + t.hy * ahy + t.hz * ahz;
-    float alx = (ahx - t.hx * hd) * t.inv_h + adj_NdL * p.nx;
-    float aly = (ahy - t.hy * hd) * t.inv_h + adj_NdL * p.ny;
-    float alz = (ahz - t.hz * hd) * t.inv_h + adj_NdL * p.nz;
-    const float adj_att0 = adj_atten * t.fall * t.s;
-    const float adj_fall = adj_atten * t.att0 * t.s;
-    const float adj_s = adj_atten * t.att0 * t.fall;
-    const float R = L.p0.w;
-    const float invR = hl_f_rcp(R);
-    float adj_d = adj_att0 * (-2.0f * t.d * t.att0 * t.att0);
-    if (t.fall > 0.0f) {
-        const float dr = t.d * invR;
-        adj_d += adj_fall * (-4.0f * dr * dr * dr * invR);
-    }
+    const float a_n = E * pn * (2.0f * (1.0f - p.a2));  // along N, through N.H
+    const float u2 = t.u * t.u;
+    const float a_p = t.hdv > 0.0f ? adj_P * (-5.0f * u2 * u2) : 0.0f;  // along V, through H.V
+    const float adj_NdL = S * t.atten + GF * t.q1 * (p.kk1 * t.inv_el - 4.0f * p.ndv * t.ndl * t.inv_den2);
+    // through H = (V + L) / |V + L|: (a - H (H.a)) / |V + L| with a = a_p V + a_n N
+    const float hd = a_p * t.hdv + a_n * t.ndh;
+    const float cV = a_p * t.inv_h, cN = a_n * t.inv_h + adj_NdL, cH = -hd * t.inv_h;
+    float alx = cH * t.hx + (cV * p.vx + cN * p.nx);
+    float aly = cH * t.hy + (cV * p.vy + cN * p.ny);
+    float alz = cH * t.hz + (cV * p.vz + cN * p.nz);
+    const float adj_atten = S * t.ndl;
+    // d(att0)/dd = -2 d att0^2 and d(fall)/dd = -4 d (d/R)^2 / R^2
+    const float r2 = L.p3.x;
+    const float dfall = t.fall > 0.0f ? 2.0f * (t.d * t.d * r2) * r2 : 0.0f;
+    const float adj_d = (-2.0f * t.d * t.att0) * (adj_atten * t.s) * (t.fall * t.att0 + dfall);
     if (L.p2.w != kNoCone && t.dsdcos != 0.0f) {
-        const float a = adj_s * t.dsdcos;
+        const float a = adj_atten * t.att0 * t.fall * t.dsdcos;
         alx -= a * L.p2.x;
         aly -= a * L.p2.y;
         alz -= a * L.p2.z;
     }
     const float ld = t.lx * alx + t.ly * aly + t.lz * alz;
-    g.x = (alx - t.lx * ld) * t.inv_d + adj_d * t.lx;
-    g.y = (aly - t.ly * ld) * t.inv_d + adj_d * t.ly;
-    g.z = (alz - t.lz * ld) * t.inv_d + adj_d * t.lz;
+    const float k = adj_d - ld * t.inv_d;
+    g.x = alx * t.inv_d + k * t.lx;
+    g.y = aly * t.inv_d + k * t.ly;
+    g.z = alz * t.inv_d + k * t.lz;
 }
 
 // -------------------------------------------------------------- block tile
@@ -302,11 +299,11 @@ __device__ __forceinline__ void ambient_terms(const ShadeArgs& a, const Pixel& p
 }
 
 // One light's adjoint for the pixels of the lanes with mine set: the
-// per-pixel gradients go to dA, dR, dM; the light's position and intensity
-// gradients, summed over the wave, to its slot copy `slot` (FP64 atomics by
-// lanes 0..3).  gl is dL/d(radiance) of the lane's pixel.
+// per-pixel sums go to m; the light's position and intensity gradients, summed
+// over the wave, to its slot copy `slot` (FP64 atomics by lanes 0..3).  gl is
+// dL/d(radiance) of the lane's pixel.
 __device__ __forceinline__ void adjoint_light(const ShadeArgs& a, const HotLight& L, uint32_t li, bool mine,
-                                              const Pixel& p, const float gl[3], float dA[3], float& dR, float& dM,
+                                              const Pixel& p, const float gl[3], float cv, MaterialSums& m,
                                               uint32_t slot) {
     const uint32_t lane = hl_lane();
     float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -314,14 +311,15 @@ __device__ __forceinline__ void adjoint_light(const ShadeArgs& a, const HotLight
     if (mine) {
         Term t;
         act = eval_term<true>(L, p, t);
-        if (act) adjoint_term(L, p, t, gl, dA, dR, dM, g);
+        if (act) adjoint_term(L, p, t, gl, cv, m, g);
     }
     if (hl_ballot(act) == 0) return;
-    const float sx = dpp_sum(g.x), sy = dpp_sum(g.y), sz = dpp_sum(g.z), si = dpp_sum(g.w);
-    if (lane < 4u) {
-        const float v = lane == 0u ? sx : (lane == 1u ? sy : (lane == 2u ? sz : si));
-        atomicAdd(a.d_light + 4 * ((size_t)slot * a.num_lights + li) + lane, (double)v);
-    }
+    const float v = dpp_sum4(g.x, g.y, g.z, g.w);
+    // color = (color * intensity) / intensity: an active term has radiance
+    // >= 0.002, hence intensity != 0
+    if (lane < 4u)
+        atomicAdd(a.d_light + 4 * ((size_t)slot * a.num_lights + li) + lane,
+                  (double)(lane == 3u ? v * hl_f_rcp(L.p3.y) : v));
 }
 
 // How the forward mode divides a view that forward_split holds for.  kOwn: the
@@ -529,15 +527,18 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
         gl[1] = g.y;
         gl[2] = g.z;
     }
-    float dA[3] = {0.0f, 0.0f, 0.0f}, dR = 0.0f, dM = 0.0f;
+    MaterialSums ms;
+    const float cv = (1.0f - p.ndv) * hl_f_rcp(p.ev);
     // per-light gradients go to one of kGradSlots copies (by wave) so that the
     // FP64 atomics of many waves on one light do not serialise on one address
     const uint32_t slot = (b * 4u + wave) % kGradSlots;
     uint32_t ord = 0;
     walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t li, bool mine) {
         if ((ord++ & 3u) != wave) return;
-        adjoint_light(a, L, li, mine, p, gl, dA, dR, dM, slot);
+        adjoint_light(a, L, li, mine, p, gl, cv, ms, slot);
     });
+    float dA[3], dR, dM;
+    adjoint_pixel(p, ms, dA, dR, dM);
     // the waves' partial per-pixel gradients, added in wave order
     float (*red)[5][64] = as->red[0];
     red[wave][0][lane] = dA[0];
@@ -640,22 +641,25 @@ __device__ __forceinline__ void fused_tile_split(const ShadeArgs& a, uint32_t b,
     if (lane == 0 && lead) atomicAdd(a.loss, (double)wl);
 
     // ---- adjoint: the same lights per wave, from LDS when they were kept
-    float dA[3] = {0.0f, 0.0f, 0.0f}, dR = 0.0f, dM = 0.0f;
+    MaterialSums ms;
+    const float cv = (1.0f - p.ndv) * hl_f_rcp(p.ev);
     const uint32_t slot = (b * 4u + wave) % kGradSlots;
     if (ks.ok) {
         for (uint32_t i = wave; i < ks.n; i += 4u) {  // uniform
             const HotLight L = s_l[i];
             const uint32_t li = hl_uniform(kept.idx[i]);
             const uint64_t lanes = kept.lanes[i];
-            adjoint_light(a, L, li, ((lanes >> lane) & 1ull) != 0ull, p, gl, dA, dR, dM, slot);
+            adjoint_light(a, L, li, ((lanes >> lane) & 1ull) != 0ull, p, gl, cv, ms, slot);
         }
     } else {
         uint32_t ord2 = 0;
         walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t li, bool mine) {
             if ((ord2++ & 3u) != wave) return;
-            adjoint_light(a, L, li, mine, p, gl, dA, dR, dM, slot);
+            adjoint_light(a, L, li, mine, p, gl, cv, ms, slot);
         });
     }
+    float dA[3], dR, dM;
+    adjoint_pixel(p, ms, dA, dR, dM);
     float (*red)[5][64] = as.red[0];
     red[wave][0][lane] = dA[0];
     red[wave][1][lane] = dA[1];
@@ -744,21 +748,24 @@ __device__ __forceinline__ void fused_tile_own(const ShadeArgs& a, uint32_t b, S
     if (lane == 0) atomicAdd(a.loss, (double)wl);
 
     // ---- adjoint: the same lights, from LDS when they were kept
-    float dA[3] = {0.0f, 0.0f, 0.0f}, dR = 0.0f, dM = 0.0f;
+    MaterialSums ms;
+    const float cv = (1.0f - p.ndv) * hl_f_rcp(p.ev);
     const uint32_t slot = (b * 4u + wave) % kGradSlots;
     if (ks.ok) {
         for (uint32_t i = 0; i < ks.n; ++i) {  // uniform
             const HotLight L = s_l[i];
             const uint32_t li = hl_uniform(kept.idx[i]);
             const uint64_t lanes = kept.lanes[i];
-            adjoint_light(a, L, li, ((lanes >> lane) & 1ull) != 0ull, p, gl, dA, dR, dM, slot);
+            adjoint_light(a, L, li, ((lanes >> lane) & 1ull) != 0ull, p, gl, cv, ms, slot);
         }
     } else {
         walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t li, bool mine) {
-            adjoint_light(a, L, li, mine, p, gl, dA, dR, dM, slot);
+            adjoint_light(a, L, li, mine, p, gl, cv, ms, slot);
         });
     }
     if (valid) {
+        float dA[3], dR, dM;
+        adjoint_pixel(p, ms, dA, dR, dM);
         const hl_gptr<float> dp = hl_g(a.d_pixel);
 #pragma unroll
         for (int c = 0; c < 3; ++c) dp[c * plane + pix] = dA[c] + gl[c] * mixv[c] * p.ao;
