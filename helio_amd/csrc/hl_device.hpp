@@ -570,42 +570,9 @@ __device__ __forceinline__ int hl_fkey(float x) {
 }
 __device__ __forceinline__ float hl_funkey(int k) { return __int_as_float(k ^ ((k >> 31) & 0x7fffffff)); }
 
-// Full-wave reductions: quad swaps, half-row and row mirrors, then the
-// row_bcast:15 / row_bcast:31 steps; lane 63 holds the result, which is read
-// back as a wave-uniform value.  All 64 lanes must be active.  Integer min/max
-// with their identity as the DPP "old" operand fold each step into one
-// v_min_i32_dpp / v_max_i32_dpp (float min/max would add a move, a NaN
-// quieting max and hazard nops per step).
-__device__ __forceinline__ int dpp_min_key(int v) {
-    constexpr int I = 0x7fffffff;
-    v = min(v, hl_dpp_i<0xB1>(I, v));
-    v = min(v, hl_dpp_i<0x4E>(I, v));
-    v = min(v, hl_dpp_i<0x141>(I, v));
-    v = min(v, hl_dpp_i<0x140>(I, v));
-    v = min(v, hl_dpp_i<0x142, 0xA>(I, v));
-    v = min(v, hl_dpp_i<0x143, 0xC>(I, v));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int dpp_max_key(int v) {
-    constexpr int I = (int)0x80000000;
-    v = max(v, hl_dpp_i<0xB1>(I, v));
-    v = max(v, hl_dpp_i<0x4E>(I, v));
-    v = max(v, hl_dpp_i<0x141>(I, v));
-    v = max(v, hl_dpp_i<0x140>(I, v));
-    v = max(v, hl_dpp_i<0x142, 0xA>(I, v));
-    v = max(v, hl_dpp_i<0x143, 0xC>(I, v));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-// min / max over the lanes with `take` set (+inf / -inf when none); inputs
-// must not be NaN.
-__device__ __forceinline__ float dpp_min_if(bool take, float v) {
-    return hl_funkey(dpp_min_key(take ? hl_fkey(v) : 0x7fffffff));
-}
-__device__ __forceinline__ float dpp_max_if(bool take, float v) {
-    return hl_funkey(dpp_max_key(take ? hl_fkey(v) : (int)0x80000000));
-}
-__device__ __forceinline__ float dpp_min(float v) { return dpp_min_if(true, v); }
-__device__ __forceinline__ float dpp_max(float v) { return dpp_max_if(true, v); }
+// Full-wave sum: quad swaps, half-row and row mirrors, then the row_bcast:15 /
+// row_bcast:31 steps; lane 63 holds the result, which is read back as a
+// wave-uniform value.  All 64 lanes must be active.
 __device__ __forceinline__ float dpp_sum(float v) {
     v = v + hl_dpp<0xB1>(0.0f, v);
     v = v + hl_dpp<0x4E>(0.0f, v);
@@ -632,6 +599,41 @@ __device__ __forceinline__ float dpp_sum4(float v0, float v1, float v2, float v3
     e = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(e), __float_as_uint(e), false, false);
     return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+}
+
+// min and max of three coordinates over the lanes with `take` set (+inf / -inf
+// when none; no NaN).  The six keys (a maximum as the minimum of complements)
+// halve with the lanes in the first three steps, as in dpp_sum4: lane bit 0
+// picks minimum or maximum, bit 1 x or y, bit 2 those or z: 13 VALU
+// instructions fewer than six reductions.  Integer keys with their identity as
+// the DPP "old" operand fold a step into one v_min_i32_dpp (float min/max would
+// add a move, a NaN quieting max and hazard nops per step).
+__device__ __forceinline__ void dpp_box_if(bool take, float x, float y, float z, float lo[3], float hi[3]) {
+    constexpr int I = 0x7fffffff;
+    const uint32_t lane = hl_lane();
+    const int flip = (lane & 1u) ? -1 : 0;
+    const float v[3] = {x, y, z};
+    int k[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int key = hl_fkey(v[c]) ^ flip;
+        k[c] = min(take ? key : I, hl_dpp_i<0xB1>(I, take ? ~key : I));  // quad_perm [1,0,3,2]
+    }
+    const bool b1 = (lane & 2u) != 0u, b2 = (lane & 4u) != 0u;
+    const int xy = min(b1 ? k[1] : k[0], hl_dpp_i<0x4E>(I, b1 ? k[0] : k[1]));  // quad_perm [2,3,0,1]
+    const int zz = min(k[2], hl_dpp_i<0x4E>(I, k[2]));
+    int e = min(b2 ? zz : xy, hl_dpp_i<0x124>(I, b2 ? xy : zz));  // row_ror:4
+    e = min(e, hl_dpp_i<0x128>(I, e));                  // row_ror:8
+    const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)e, (uint32_t)e, false, false);
+    e = min((int)r[0], (int)r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)e, (uint32_t)e, false, false);
+    e = min((int)h[0], (int)h[1]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int lane0 = c == 0 ? 0 : (c == 1 ? 2 : 4);
+        lo[c] = hl_funkey(__builtin_amdgcn_readlane(e, lane0));
+        hi[c] = hl_funkey(~__builtin_amdgcn_readlane(e, lane0 + 1));
+    }
 }
 
 // Placed in a rarely taken block, keeps the optimizer from executing the block
