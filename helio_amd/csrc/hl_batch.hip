@@ -1,7 +1,8 @@
 // hl_batch.hip -- batched multi-view frames: one plan holds many views (probe
 // cube faces, XR eyes) over a shared light pool.  A frame is a fixed sequence
 // of launches that each cover every view:
-//   light gather + clustered cull (k_batch_prep/geom/mark/count/scan/fill),
+//   light gather + clustered cull (k_batch_col_*, and k_batch_* for the views
+//   whose grids are too large for it),
 //   one persistent shading launch over a heaviest-first queue of
 //   (view, block tile) items (forward, or forward + L2 adjoint per view),
 //   per-light gradient write-back for the adjoint views;
@@ -42,8 +43,17 @@ struct ViewBufs {
     void* counts = nullptr;
     void* pool = nullptr;
     void* acc = nullptr;
+    void* columns = nullptr;  // column path only (geom, bits and summary: mark path only)
     uint32_t pool_cap = 0;
 };
+
+// Blocks the column path's views share, and its scratch over a plan.
+// 512 blocks are aimed at: whole columns on all but the smallest grids, where
+// a few blocks per view are enough (256 and 1024 measured the same for a frame
+// of 24 faces and two eyes: 24.1 and 25.8 us counting, against 24.2).  1 GiB holds the scratch of the 50-view frame of 48 faces and two
+// 2064x2208 eyes four times over.
+constexpr uint32_t kBatchColBlocks = 512;
+constexpr size_t kBatchColScratch = 1ull << 30;
 
 }  // namespace
 
@@ -62,7 +72,12 @@ struct hl_plan {
     BatchShadeView* d_shade = nullptr;
     uint32_t* d_light_base = nullptr;
     uint32_t* d_cell_base = nullptr;
-    uint32_t* d_tile_base = nullptr;
+    // views on the column path: records, first prep and column blocks
+    void* d_cols = nullptr;
+    uint32_t* d_prep_base = nullptr;
+    uint32_t* d_col_base = nullptr;
+    std::vector<uint32_t> col_views, col_aim, mark_views;
+    uint32_t prep_blocks = 0, col_blocks = 0;
     uint2* d_spans = nullptr;  // per group: (first item, view) per view + (item count, 0)
     uint32_t* d_queue = nullptr;
     uint32_t* d_flags = nullptr;
@@ -72,7 +87,7 @@ struct hl_plan {
     GradView* d_grad = nullptr;
     uint32_t num_grad = 0, grad_max_n = 0;
     size_t grad_words = 0;
-    uint32_t total_lights = 0, total_cells = 0, total_tiles = 0, num_items = 0;
+    uint32_t total_lights = 0, total_cells = 0, num_items = 0;  // lights, cells: the mark path's views
     // shading items grouped by (G-buffer format set, mode): one persistent
     // launch per non-empty group; group = set * 2 + (adjoint ? 1 : 0)
     uint32_t grp_first[6] = {}, grp_spans[6] = {}, grp_count[6] = {}, grp_grid[6] = {};
@@ -98,7 +113,7 @@ hl_status plan_alloc(hl_plan* p, void** out, size_t bytes, bool zero = false) {
 
 void free_bufs(ViewBufs& b) {
     for (void** q : {&b.hot, &b.cull, &b.geom, &b.bits, &b.summary, &b.raw, &b.offsets, &b.counts,
-                     &b.pool, &b.acc})
+                     &b.pool, &b.acc, &b.columns})
         if (*q) {
             (void)hipFree(*q);
             *q = nullptr;
@@ -108,13 +123,13 @@ void free_bufs(ViewBufs& b) {
 void free_plan_device(hl_plan* p) {
     for (auto& b : p->bufs) free_bufs(b);
     for (void* q : {(void*)p->d_cull, (void*)p->d_shade, (void*)p->d_light_base, (void*)p->d_cell_base,
-                    (void*)p->d_tile_base,
+                    p->d_cols, (void*)p->d_prep_base, (void*)p->d_col_base,
                     (void*)p->d_spans, (void*)p->d_queue, (void*)p->d_flags, p->d_markq})
         if (q) (void)hipFree(q);
-    p->d_markq = nullptr;
+    p->d_markq = p->d_cols = nullptr;
     p->d_cull = nullptr;
     p->d_shade = nullptr;
-    p->d_light_base = p->d_cell_base = p->d_tile_base = p->d_queue = p->d_flags = nullptr;
+    p->d_light_base = p->d_cell_base = p->d_prep_base = p->d_col_base = p->d_queue = p->d_flags = nullptr;
     p->d_spans = nullptr;
     if (p->exec) (void)hipGraphExecDestroy(p->exec);
     if (p->graph) (void)hipGraphDestroy(p->graph);
@@ -130,15 +145,41 @@ double block_cost(const hl_plan* p, uint32_t v) {
     return (is_adjoint(p->views[v]) ? 4.0 : 1.0) * (1.0 + log2(1.0 + lights));
 }
 
+// The culls of every view.  Their first kernels clear the views' overflow
+// words.
+hl_status enqueue_cull(hl_plan* p, hipStream_t s) {
+    hl_context* c = p->ctx;
+    HL_HIP(c, launch_batch_columns(s, p->d_cols, p->d_prep_base, p->d_col_base, (uint32_t)p->col_views.size(),
+                                   p->prep_blocks, p->col_blocks));
+    HL_HIP(c, launch_batch_cull(s, p->pool, p->d_cull, p->d_light_base, p->d_cell_base,
+                                (uint32_t)p->mark_views.size(), p->total_lights, p->total_cells,
+                                mark_queue_at(p->d_markq, p->total_lights)));
+    return HL_OK;
+}
+
+// The views' cull records (again after a list pool has grown).
+hl_status upload_cull(hl_plan* p) {
+    hl_context* c = p->ctx;
+    std::vector<BatchCullView> marks;
+    for (uint32_t v : p->mark_views) marks.push_back(p->hcull[v]);
+    if (!marks.empty())
+        HL_HIP(c, hipMemcpy(p->d_cull, marks.data(), sizeof(BatchCullView) * marks.size(), hipMemcpyHostToDevice));
+    const size_t rec = batch_column_view_size();
+    std::vector<uint8_t> cols(rec * p->col_views.size());
+    for (size_t i = 0; i < p->col_views.size(); ++i) {
+        const uint32_t v = p->col_views[i];
+        batch_column_view(cols.data() + rec * i, p->hcull[v], p->pool, p->bufs[v].columns, p->col_aim[i]);
+    }
+    if (!cols.empty()) HL_HIP(c, hipMemcpy(p->d_cols, cols.data(), cols.size(), hipMemcpyHostToDevice));
+    return HL_OK;
+}
+
 hl_status enqueue_frame(hl_plan* p, hipStream_t s) {
     hl_context* c = p->ctx;
-    const uint32_t nv = (uint32_t)p->views.size();
     HL_HIP(c, launch_grad_views_zero(s, p->d_grad, p->num_grad, p->grad_words));
-    // the cull's first kernel clears the views' overflow words; the shading
-    // launches leave their claim counters zero for the next frame
-    HL_HIP(c, launch_batch_cull(s, p->pool, p->d_cull, p->d_light_base, p->d_cell_base,
-                                p->d_tile_base, nv, p->total_lights, p->total_cells, p->total_tiles,
-                                mark_queue_at(p->d_markq, p->total_lights)));
+    // the shading launches leave their claim counters zero for the next frame
+    const hl_status cs = enqueue_cull(p, s);
+    if (cs != HL_OK) return cs;
     for (int g = 0; g < 6; ++g)
         HL_HIP(c, launch_shade_batch(s, g / 2, (g & 1) ? kModeFusedL2 : kModeForward, p->d_shade,
                                      p->d_spans + p->grp_first[g], p->grp_spans[g], p->grp_count[g],
@@ -156,7 +197,10 @@ hl_status build_plan(hl_plan* p) {
     p->bufs.assign(nv, ViewBufs{});
     p->hcull.assign(nv, BatchCullView{});
     p->hshade.assign(nv, BatchShadeView{});
-    std::vector<uint32_t> light_base(nv + 1, 0), cell_base(nv + 1, 0), tile_base(nv + 1, 0);
+    std::vector<uint32_t> light_base(1, 0), cell_base(1, 0), prep_base(1, 0), col_base(1, 0);
+    p->col_views.clear();
+    p->col_aim.clear();
+    p->mark_views.clear();
     hl_status s;
     if ((s = plan_alloc(p, (void**)&p->d_flags, 4 * (size_t)nv)) != HL_OK) return s;
     for (uint32_t v = 0; v < nv; ++v) {
@@ -179,6 +223,21 @@ hl_status build_plan(hl_plan* p) {
             const hl_status st = check_cluster_params(c, &cp);
             if (st != HL_OK) return st;
         }
+    }
+    // The column path's blocks are shared out by cells x lights.  Its scratch
+    // (12 bytes per block and light) is bounded over the plan: views past
+    // kBatchColScratch keep the mark path.
+    double work = 0.0;
+    const auto view_work = [&](uint32_t v) {
+        const hl_cluster_params& cp = p->cparams[v];
+        return (double)cp.grid_x * cp.grid_y * cp.grid_z * (p->nlights[v] + 1.0);
+    };
+    for (uint32_t v = 0; v < nv; ++v) work += view_work(v);
+    size_t col_scratch = 0;
+    uint64_t lights = 0, cells = 0;  // of all views
+    for (uint32_t v = 0; v < nv; ++v) {
+        const hl_view_desc& d = p->views[v];
+        const hl_cluster_params& cp = p->cparams[v];
         static_assert(HL_BATCH_MAX_VIEWS < 256u, "view index of a mark queue entry: 8 bits");
         static_assert((1u << 26) / 64u < (1u << 24), "chunk index of a mark queue entry: 24 bits");
         const uint32_t n = p->nlights[v];
@@ -186,9 +245,17 @@ hl_status build_plan(hl_plan* p) {
         ViewBufs& b = p->bufs[v];
         if ((s = plan_alloc(p, &b.hot, sizeof(HotLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
         if ((s = plan_alloc(p, &b.cull, sizeof(CullLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
-        if ((s = plan_alloc(p, &b.geom, cluster_geom_bytes(ncol, ncell))) != HL_OK) return s;
-        if ((s = plan_alloc(p, &b.bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
-        if ((s = plan_alloc(p, &b.summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;
+        const uint32_t aim = (uint32_t)(kBatchColBlocks * (view_work(v) / work)) + 1u;
+        const BatchColumnPlan col = batch_column_plan(cp.grid_x, cp.grid_y, cp.grid_z, n, aim);
+        const bool columns = col.blocks != 0 && col_scratch + col.scratch <= kBatchColScratch;
+        if (columns) {
+            if ((s = plan_alloc(p, &b.columns, col.scratch)) != HL_OK) return s;
+            col_scratch += col.scratch;
+        } else {
+            if ((s = plan_alloc(p, &b.geom, cluster_geom_bytes(ncol, ncell))) != HL_OK) return s;
+            if ((s = plan_alloc(p, &b.bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
+            if ((s = plan_alloc(p, &b.summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;
+        }
         if ((s = plan_alloc(p, &b.raw, cluster_raw_bytes(ncell))) != HL_OK) return s;
         if ((s = plan_alloc(p, &b.offsets, 4 * (size_t)ncell)) != HL_OK) return s;
         if ((s = plan_alloc(p, &b.counts, 4 * (size_t)ncell)) != HL_OK) return s;
@@ -216,37 +283,46 @@ hl_status build_plan(hl_plan* p) {
         cv.W = (n + 31u) / 32u;
         cv.SW = (cv.W + 31u) / 32u;
         cv.ncell = ncell;
-        if ((uint64_t)light_base[v] + n >= (1ull << 28) ||
-            (uint64_t)cell_base[v] + ncell + kBatchCellAlign >= (1ull << 31))
+        const uint32_t cells_v = (ncell + kBatchCellAlign - 1u) / kBatchCellAlign * kBatchCellAlign;
+        if (lights + n >= (1ull << 28) || cells + ncell + kBatchCellAlign >= (1ull << 31))
             return fail(c, HL_ECAPACITY, "plan too large: %u views up to view %u exceed 2^28 lights or 2^31 cells",
                         nv, v);
-        light_base[v + 1] = light_base[v] + n;
-        cell_base[v + 1] = cell_base[v] + (ncell + kBatchCellAlign - 1u) / kBatchCellAlign * kBatchCellAlign;
-        tile_base[v + 1] = tile_base[v] + cluster_scan_tiles(ncell);
+        lights += n;
+        cells += cells_v;
+        if (columns) {
+            p->col_views.push_back(v);
+            p->col_aim.push_back(aim);
+            prep_base.push_back(prep_base.back() + col.prep_blocks);
+            col_base.push_back(col_base.back() + col.blocks);
+        } else {
+            p->mark_views.push_back(v);
+            light_base.push_back(light_base.back() + n);
+            cell_base.push_back(cell_base.back() + cells_v);
+        }
     }
-    p->total_lights = light_base[nv];
-    p->total_cells = cell_base[nv];
-    p->total_tiles = tile_base[nv];
-    if ((s = plan_alloc(p, (void**)&p->d_cull, sizeof(BatchCullView) * nv)) != HL_OK) return s;
-    if ((s = plan_alloc(p, (void**)&p->d_light_base, 4 * (size_t)(nv + 1))) != HL_OK) return s;
-    if ((s = plan_alloc(p, (void**)&p->d_cell_base, 4 * (size_t)(nv + 1))) != HL_OK) return s;
+    p->total_lights = light_base.back();
+    p->total_cells = cell_base.back();
+    p->prep_blocks = prep_base.back();
+    p->col_blocks = col_base.back();
+    if ((s = plan_alloc(p, (void**)&p->d_cull, sizeof(BatchCullView) * p->mark_views.size())) != HL_OK) return s;
+    if ((s = plan_alloc(p, &p->d_cols, batch_column_view_size() * p->col_views.size())) != HL_OK) return s;
     if ((s = plan_alloc(p, &p->d_markq, mark_queue_bytes(p->total_lights))) != HL_OK) return s;
-    if ((s = plan_alloc(p, (void**)&p->d_tile_base, 4 * (size_t)(nv + 1))) != HL_OK) return s;
-    HL_HIP(c, hipMemcpy(p->d_tile_base, tile_base.data(), 4 * (nv + 1), hipMemcpyHostToDevice));
-    HL_HIP(c, hipMemcpy(p->d_light_base, light_base.data(), 4 * (nv + 1), hipMemcpyHostToDevice));
-    HL_HIP(c, hipMemcpy(p->d_cell_base, cell_base.data(), 4 * (nv + 1), hipMemcpyHostToDevice));
+    const std::pair<uint32_t**, const std::vector<uint32_t>*> bases[] = {
+        {&p->d_light_base, &light_base}, {&p->d_cell_base, &cell_base}, {&p->d_prep_base, &prep_base}, {&p->d_col_base, &col_base}};
+    for (const auto& b : bases) {
+        if ((s = plan_alloc(p, (void**)b.first, 4 * b.second->size())) != HL_OK) return s;
+        HL_HIP(c, hipMemcpy(*b.first, b.second->data(), 4 * b.second->size(), hipMemcpyHostToDevice));
+    }
     // size each pool from a first cull: exact totals + headroom
     for (int pass = 0; pass < 2; ++pass) {
-        HL_HIP(c, hipMemcpy(p->d_cull, p->hcull.data(), sizeof(BatchCullView) * nv, hipMemcpyHostToDevice));
+        if ((s = upload_cull(p)) != HL_OK) return s;
         HL_HIP(c, launch_fill_u32(c->stream, p->d_flags, 0, nv));
-        HL_HIP(c, launch_batch_cull(c->stream, p->pool, p->d_cull, p->d_light_base, p->d_cell_base,
-                                    p->d_tile_base, nv, p->total_lights, p->total_cells,
-                                    p->total_tiles, mark_queue_at(p->d_markq, p->total_lights)));
+        if ((s = enqueue_cull(p, c->stream)) != HL_OK) return s;
         {
             const hipError_t e = hipStreamSynchronize(c->stream);
             if (e != hipSuccess)
-                return fail(c, HL_EHIP, "plan cull pass %d (%u views, %u lights, %u clusters): %s", pass, nv,
-                            p->total_lights, p->total_cells, hipGetErrorString(e));
+                return fail(c, HL_EHIP, "plan cull pass %d (%u views, %llu lights, %llu clusters): %s", pass, nv,
+                            (unsigned long long)lights, (unsigned long long)cells, hipGetErrorString(e));
         }
         bool grew = false;
         for (uint32_t v = 0; v < nv; ++v) {
@@ -269,7 +345,7 @@ hl_status build_plan(hl_plan* p) {
         }
         if (!grew) break;
     }
-    HL_HIP(c, hipMemcpy(p->d_cull, p->hcull.data(), sizeof(BatchCullView) * nv, hipMemcpyHostToDevice));
+    if ((s = upload_cull(p)) != HL_OK) return s;
     // shading records
     std::vector<std::pair<double, uint32_t>> order;
     std::vector<int> vset(nv, 0);

@@ -1236,26 +1236,31 @@ __device__ __forceinline__ uint64_t member_slices(const ColBlock& c, const ColGe
 
 // A wave per block: the lights' chains (loads, FP64 band, bisections) over all
 // CUs rather than over n / 256 of them.
-__global__ __launch_bounds__(64) void k_col_prep(ClusterArgs a, ColumnArgs p, uint32_t nsum) {
-    __shared__ SliceTab tab;
+__device__ __forceinline__ void col_prep_block(const ClusterArgs& a, const ColumnArgs& p, uint32_t block,
+                                               uint32_t nblocks, uint32_t nsum, SliceTab& tab) {
     load_slices(a, tab);
     __syncthreads();
-    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+    const uint32_t i = block * 64u + threadIdx.x;
     if (i == 0) {
         *p.flags = 0u;
         if (p.flags2) *p.flags2 = 0u;
     }
-    for (uint32_t j = i; j < nsum; j += gridDim.x * 64u) p.gsum[j] = 0u;
+    for (uint32_t j = i; j < nsum; j += nblocks * 64u) p.gsum[j] = 0u;
     if (i >= a.num_lights) {
         if (i < ((a.num_lights + 3u) & ~3u)) p.box_col[i] = kNoBox;
         return;
     }
-    const CullLight L = cull_light_at(p.lights, i, p.cam);
+    const CullLight L = cull_light_at(p.lights, p.subset ? p.subset[i] : i, p.cam);
     p.cull[i] = L;
     const LightBox b = light_box(a, p.cam, L.vpos, L.cone.w != kNoCone, tab);
     p.box_col[i] = b.col;
     p.box_slice[i] = b.slice;
-    prep_one(p.lights, nullptr, a.num_lights, p.cam, p.hot, nullptr, p.feature_flags, i);
+    prep_one(p.lights, p.subset, a.num_lights, p.cam, p.hot, nullptr, p.feature_flags, i);
+}
+
+__global__ __launch_bounds__(64) void k_col_prep(ClusterArgs a, ColumnArgs p, uint32_t nsum) {
+    __shared__ SliceTab tab;
+    col_prep_block(a, p, blockIdx.x, gridDim.x, nsum, tab);
 }
 
 // INLINE: the block bounds every light itself (a light per thread; the cone
@@ -1581,8 +1586,106 @@ size_t column_scratch_bytes(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n) {
     return column_scratch(nullptr, ncol, gz, n, column_plan(ncol, gz, kColBlocks).blocks, nullptr);
 }
 
-// Cells of every view, then (blocks past geom_blocks) the lights of every
+// The column path of many views: the same three steps, a launch each, the
+// blocks of a view one after the other (base: first block of each view, and
+// the end).  The plan aims at a number of blocks for the whole batch, shared
+// out by cells x lights.  Lights are scanned kBatchColChunk at a time: the smaller list (8 KB against 32) lets four
+// blocks share a CU.  24 faces of 128^2 with 512 lights each and two 1032x1104
+// eyes with 4096: 7 + 23 + 8 us against the mark path's 51 (geometry 6, mark
+// 12, tail 11, count 9, fill 12).
+struct BatchColumnView {
+    ClusterArgs a;
+    ColumnArgs p;
+    uint32_t nsum, nprep;
+};
+// read through the constant address space, as k_shade_batch reads its views
+typedef const __attribute__((address_space(4))) BatchColumnView* ConstColumnViews;
+constexpr uint32_t kBatchColChunk = 4096;
+// The view of a block (base strictly ascending): every lane compares one
+// entry, one round trip instead of the bisection's log2(nviews).
+__device__ __forceinline__ uint32_t view_of_block(const uint32_t* __restrict__ base, uint32_t nviews) {
+    uint32_t v = 0;
+    for (uint32_t q = 1; q < nviews; q += 64u) {
+        const uint32_t i = q + hl_lane();
+        v += (uint32_t)__popcll(hl_ballot(i < nviews && base[i] <= blockIdx.x));
+    }
+    return hl_uniform(v);
+}
 
+__global__ __launch_bounds__(64) void k_batch_col_prep(ConstColumnViews __restrict__ views,
+                                                       const uint32_t* __restrict__ base, uint32_t nviews) {
+    __shared__ SliceTab tab;
+    const uint32_t vi = view_of_block(base, nviews);
+    const BatchColumnView& v = *(const BatchColumnView*)&views[vi];
+    col_prep_block(v.a, v.p, blockIdx.x - base[vi], v.nprep, v.nsum, tab);
+}
+
+__global__ __launch_bounds__(kColThreads) void k_batch_col_count(ConstColumnViews __restrict__ views,
+                                                                 const uint32_t* __restrict__ base, uint32_t nviews) {
+    __shared__ ColCountSmem<kBatchColChunk> sm;
+    const uint32_t vi = view_of_block(base, nviews);
+    const BatchColumnView& v = *(const BatchColumnView*)&views[vi];
+    col_count_block<kBatchColChunk, false>(v.a, v.p, blockIdx.x - base[vi], 0u, sm, nullptr);
+}
+
+__global__ __launch_bounds__(256) void k_batch_col_fill(ConstColumnViews __restrict__ views,
+                                                        const uint32_t* __restrict__ base, uint32_t nviews) {
+    __shared__ ColFillSmem sm;
+    const uint32_t vi = view_of_block(base, nviews);
+    const BatchColumnView& v = *(const BatchColumnView*)&views[vi];
+    col_fill_block<true>(v.a, v.p, blockIdx.x - base[vi], sm);
+}
+
+size_t batch_column_view_size() { return sizeof(BatchColumnView); }
+
+BatchColumnPlan batch_column_plan(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n, uint32_t aim) {
+    BatchColumnPlan r;
+    if (!use_columns(gx, gy, gz, n)) return r;
+    const ColumnPlan cp = column_plan(gx * gy, gz, aim);
+    r.blocks = cp.blocks;
+    r.prep_blocks = n ? (n + 63u) / 64u : 1u;
+    r.scratch = column_scratch(nullptr, gx * gy, gz, n, cp.blocks, nullptr);
+    return r;
+}
+
+void batch_column_view(void* dst, const BatchCullView& v, const GpuLight* pool, void* scratch, uint32_t aim) {
+    BatchColumnView& o = *(BatchColumnView*)dst;
+    const uint32_t ncol = v.ca.grid_x * v.ca.grid_y, gz = v.ca.grid_z, n = v.ca.num_lights;
+    const ColumnPlan cp = column_plan(ncol, gz, aim);
+    o.a = v.ca;
+    o.p = ColumnArgs{};
+    o.p.cam = v.cam;
+    o.p.lights = pool;
+    o.p.subset = v.subset;
+    o.p.hot = v.hot;
+    o.p.cull = v.cull;
+    o.p.raw = v.raw;
+    o.p.offsets = v.offsets;
+    o.p.counts = v.counts;
+    o.p.pool = v.pool;
+    o.p.pool_cap = v.pool_cap;
+    o.p.kb = cp.kb;
+    o.p.flags = v.flags;
+    (void)column_scratch((uint8_t*)scratch, ncol, gz, n, cp.blocks, &o.p);
+    o.nsum = column_groups(ncol) * gz;
+    o.nprep = n ? (n + 63u) / 64u : 1u;
+}
+
+hipError_t launch_batch_columns(hipStream_t s, const void* views, const uint32_t* prep_base, const uint32_t* col_base,
+                                uint32_t nviews, uint32_t prep_blocks, uint32_t col_blocks) {
+    if (nviews == 0) return hipSuccess;
+    const ConstColumnViews v = (ConstColumnViews)views;
+    hipError_t e;
+    k_batch_col_prep<<<prep_blocks, 64, 0, s>>>(v, prep_base, nviews);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    k_batch_col_count<<<col_blocks, kColThreads, 0, s>>>(v, col_base, nviews);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    k_batch_col_fill<<<col_blocks, 256, 0, s>>>(v, col_base, nviews);
+    return hipGetLastError();
+}
+
+// The mark path of many views.
+// Cells of every view, then (blocks past geom_blocks) the lights of every
 // view gathered from the pool, in one launch.
 __global__ __launch_bounds__(256) void k_batch_geom(const BatchCullView* __restrict__ views,
                                                     const uint32_t* __restrict__ cell_base,
@@ -1677,9 +1780,9 @@ __global__ __launch_bounds__(256) void k_batch_fill(const BatchCullView* __restr
 static uint32_t tail_blocks(uint32_t) { return 16u * kMarkQueues; }
 
 hipError_t launch_batch_cull(hipStream_t s, const GpuLight* pool, const BatchCullView* views,
-                             const uint32_t* light_base, const uint32_t* cell_base,
-                             const uint32_t* tile_base, uint32_t nviews, uint32_t total_lights,
-                             uint32_t total_cells, uint32_t total_tiles, const MarkQueue& mq) {
+                             const uint32_t* light_base, const uint32_t* cell_base, uint32_t nviews,
+                             uint32_t total_lights, uint32_t total_cells, const MarkQueue& mq) {
+    if (nviews == 0) return hipSuccess;
     if (total_cells % kBatchCellAlign) return hipErrorInvalidValue;
     hipError_t e;
     const uint32_t geom_blocks = total_cells / 256u;  // total_cells: kBatchCellAlign multiple

@@ -186,10 +186,23 @@ struct BatchCullView {
     uint32_t* flags;
     uint32_t pool_cap, W, SW, ncell;
 };
+// the views whose grids take the mark path
 hipError_t launch_batch_cull(hipStream_t s, const GpuLight* pool, const BatchCullView* views,
-                             const uint32_t* light_base, const uint32_t* cell_base,
-                             const uint32_t* tile_base, uint32_t nviews, uint32_t total_lights,
-                             uint32_t total_cells, uint32_t total_tiles, const MarkQueue& mq);
+                             const uint32_t* light_base, const uint32_t* cell_base, uint32_t nviews,
+                             uint32_t total_lights, uint32_t total_cells, const MarkQueue& mq);
+
+// The views whose grids take the column path: `aim` blocks are aimed at for a
+// view; blocks == 0 when its grid takes the mark path.  batch_column_view fills
+// a record of batch_column_view_size() bytes.
+struct BatchColumnPlan {
+    uint32_t blocks = 0, prep_blocks = 0;
+    size_t scratch = 0;
+};
+BatchColumnPlan batch_column_plan(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n, uint32_t aim);
+size_t batch_column_view_size();
+void batch_column_view(void* dst, const BatchCullView& v, const GpuLight* pool, void* scratch, uint32_t aim);
+hipError_t launch_batch_columns(hipStream_t s, const void* views, const uint32_t* prep_base, const uint32_t* col_base,
+                                uint32_t nviews, uint32_t prep_blocks, uint32_t col_blocks);
 
 // Prepares the lights' records (hot: shading, may be null; cl: culling; feature
 // flags) and builds the lists.

@@ -80,7 +80,8 @@ def test_batch_equals_single(ctx, hlib):
             ids = np.arange(first, first + len(sc.lights), dtype=np.uint32)
             views.append(BatchView(scene=upload_scene(ctx, sc), subset=ctx.upload(ids), num_lights=len(ids),
                                    out=ctx.alloc(sc.width * sc.height * 16)))
-        plan = BatchPlan(ctx, ctx.upload(pool), len(pool), views)
+        pool_d = ctx.upload(pool)  # the plan reads it at every launch
+        plan = BatchPlan(ctx, pool_d, len(pool), views)
         try:
             for v in views:
                 v.out.fill_u32(0)
