@@ -241,6 +241,20 @@ constexpr int kModeMask = 7;
 constexpr uint32_t kFusedSplitBlocks = 4096;
 __host__ __device__ inline bool fused_split(uint32_t num_blocks) { return num_blocks < kFusedSplitBlocks; }
 
+// Waves that share a wave tile in the backward mode, as a power of two: four
+// give a small view enough waves and cut the longest chains, but each repeats
+// the tile's set-up and walk.  Whole backward calls, us, with 4 / 2 / 1 waves, by
+// block tiles and lights: 256 36 / 40 / 44 (64 lights), 62 / 77 / 112 (512);
+// 1024 51 / 44 / 47, 82 / 83 / 111; 1350 61 / 53 / 54, 91 / 101 / 128; 2304
+// 79 / 57 / 55, 113 / 95 / 108; 3072 100 / 70 / 52, 156 / 124 / 116; 5120
+// 137 / 85 / 63, 201 / 140 / 138.  (The fused step keeps four up to its bound
+// above: its loss is returned in 64 bits, and other shares would move it by the
+// rounding of the radiance.)
+__host__ __device__ inline uint32_t backward_share(uint32_t num_blocks, uint32_t num_lights) {
+    if (num_blocks < 2048u && (num_blocks <= 512u || num_blocks <= 3ull * num_lights)) return 2u;
+    return num_blocks < 2560u ? 1u : 0u;
+}
+
 // The forward mode shares a wave tile's lights among the block's four waves, by
 // the light's index modulo 4, on small views and on views that are small for
 // their lights: a 128^2 view has 256 wave tiles for 1024 SIMDs, and a wave that
@@ -258,14 +272,15 @@ __host__ __device__ inline bool forward_split(uint32_t width, uint32_t height, u
 }
 
 // Work items of a single-view shading launch of MODE (a ShadeMode with its
-// flags): the backward mode, the shared forward and the fused mode when split
-// share each wave tile's lights among a block's four waves, so their items are
-// wave tiles (four per block tile).  A batched launch shares under the fused
+// flags): the shared forward and the fused mode when split share each wave
+// tile's lights among a block's four waves, so their items are wave tiles (four
+// per block tile), and the backward mode likewise by its share.  A batched launch shares under the fused
 // mode only.
 template <int MODE>
 __host__ __device__ inline uint32_t shade_items(const ShadeArgs& a) {
     constexpr int M = MODE & kModeMask;
-    const bool split = M == kModeBackward || (MODE & kModeShared) || (M == kModeFusedL2 && fused_split(a.num_blocks));
+    if (M == kModeBackward) return a.num_blocks << backward_share(a.num_blocks, a.num_lights);
+    const bool split = (MODE & kModeShared) || (M == kModeFusedL2 && fused_split(a.num_blocks));
     return split ? 4u * a.num_blocks : a.num_blocks;
 }
 

@@ -339,12 +339,12 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     b = hl_uniform(b);  // the item is the block's: its tile arithmetic stays scalar
     const uint32_t lane = threadIdx.x & 63u, wave = hl_uniform(threadIdx.x >> 6);
     constexpr bool kAdj = MODE == kModeBackward;
-    // The backward mode splits a wave tile's adjoint over the block's four
-    // waves (every fourth light each; the items are wave tiles, four per block
-    // tile): its per-light work is several times the forward's, and the
-    // heaviest tiles would otherwise set the launch's length.  The forward
-    // mode shares a wave tile's lights alike under kShare; else each wave has
-    // its own tile of the block tile.
+    // The backward mode splits a wave tile's adjoint over up to four waves of
+    // the block by the ordinals of its lights (backward_share): its per-light
+    // work is several times the forward's, and on small views the heaviest tiles
+    // would otherwise set the launch's length.  The forward mode shares a wave
+    // tile's lights alike under kShare; else each wave has its own tile of the
+    // block tile.
     constexpr bool kRC = MODE == kModeExtended;
     constexpr bool kExt = MODE == kModeShadowed || kRC;  // exact N, shadow_factor
     constexpr bool kFwd = MODE == kModeForward || kExt;
@@ -354,14 +354,18 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
         MODE == kModeForward && DIV == kClasses && forward_split(a.width, a.height, a.num_lights);
     const uint32_t twl = a.tw_log2, tw = 1u << twl;
     const uint32_t th = 64u >> twl;
-    const uint32_t bt = split ? b >> 2 : b, sub = split ? (b & 3u) : wave;
+    // 2^sh waves share a tile; this one is number part_no of them, and the block
+    // holds 4 >> sh tiles
+    const uint32_t sh = kAdj ? backward_share(a.num_blocks, a.num_lights) : (split ? 2u : 0u);
+    const uint32_t share = (1u << sh) - 1u, part_no = wave & share;
+    const uint32_t bt = b >> sh, sub = ((b & share) << (2u - sh)) + (wave >> sh);
     const uint32_t bx = bt % a.block_tiles_x, by = bt / a.block_tiles_x;
     const uint32_t x = bx * (4u * tw) + sub * tw + (lane & (tw - 1u));
     const uint32_t y = by * th + (lane >> twl);
     const bool inside = x < a.width && y < a.height;
     const float depth = inside ? hl_load_depth(a.depth, x, y) : 1.0f;
     const bool valid = inside && depth < 1.0f;
-    const bool lead = !split || wave == 0u;  // writes the tile's shared results
+    const bool lead = part_no == 0u;  // writes the tile's shared results
     constexpr bool kWrites = kFwd;
     // the pixel's address, computed once (8 B per pixel for RGBA16F, else 16)
     constexpr bool out_f16 = F16;
@@ -376,7 +380,13 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
         if (kAdj)
             for (int k = 0; k < HL_PIXEL_GRAD_PLANES; ++k) hl_g(a.d_pixel)[k * plane + pix] = 0.0f;
     }
-    if (hl_ballot(valid) == 0) return;
+    if (hl_ballot(valid) == 0) {
+        if (kAdj) {  // the block's other tile may hold pixels: its waves meet twice
+            __syncthreads();
+            __syncthreads();
+        }
+        return;
+    }
 
     // ---- per-pixel set-up (deferred_lighting.wgsl:999-1086)
     Pixel p;
@@ -534,7 +544,7 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     const uint32_t slot = (b * 4u + wave) % kGradSlots;
     uint32_t ord = 0;
     walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t li, bool mine) {
-        if ((ord++ & 3u) != wave) return;
+        if ((ord++ & share) != part_no) return;
         adjoint_light(a, L, li, mine, p, gl, cv, ms, slot);
     });
     float dA[3], dR, dM;
@@ -547,10 +557,14 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     red[wave][3][lane] = dR;
     red[wave][4][lane] = dM;
     __syncthreads();
+    if (lead) {
+        for (uint32_t w = wave + 1u; w <= wave + share; ++w) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) dA[c] = ((red[0][c][lane] + red[1][c][lane]) + red[2][c][lane]) + red[3][c][lane];
-    dR = ((red[0][3][lane] + red[1][3][lane]) + red[2][3][lane]) + red[3][3][lane];
-    dM = ((red[0][4][lane] + red[1][4][lane]) + red[2][4][lane]) + red[3][4][lane];
+            for (int c = 0; c < 3; ++c) dA[c] += red[w][c][lane];
+            dR += red[w][3][lane];
+            dM += red[w][4][lane];
+        }
+    }
     __syncthreads();
     if (valid && lead) {
 #pragma unroll
