@@ -267,6 +267,14 @@ struct KeptState {
 struct LightShare {
     uint32_t mask = 0u, value = 0u;
 };
+// Waves that share a tile by the ordinals of its visited lights: f is called,
+// and with kept a record stored, only where ord % (mask + 1) == value.  The
+// lights of the other waves cost a bit of the ballot here, no staging and no
+// turn of the loop (512^2 fused step 85 -> 80 us a call, 773x431 backward 91 -> 87).
+struct OrdinalShare {
+    uint32_t mask, value;
+    uint32_t ord = 0u;  // lights visited so far
+};
 struct OneClass {
     static constexpr bool kOne = true;
 };
@@ -279,7 +287,8 @@ struct LightClasses {
 template <int GRID, bool kKeep = false, class A, class F, class C = OneClass>
 __device__ __forceinline__ void walk_lights(const A& a, HotLight* s_l, const Pixel& p, bool valid,
                                             uint32_t cell, F&& f, KeptLights* kept = nullptr,
-                                            KeptState* ks = nullptr, LightShare share = LightShare{}, C&& classes = C{}) {
+                                            KeptState* ks = nullptr, LightShare share = LightShare{}, C&& classes = C{},
+                                            OrdinalShare* turns = nullptr) {
     const uint32_t lane = hl_lane();
     uint64_t todo = hl_ballot(valid);
     while (todo) {
@@ -334,6 +343,12 @@ __device__ __forceinline__ void walk_lights(const A& a, HotLight* s_l, const Pix
                 }
             }
             uint64_t m = hl_ballot(pass);
+            if (turns) {
+                const uint32_t ord = turns->ord + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                turns->ord += (uint32_t)__popcll(m);
+                pass = pass && (ord & turns->mask) == turns->value;
+                m = hl_ballot(pass);
+            }
             // kKeep: the kept range's next slots in lane order while they fit,
             // else the lane's own
             bool keep = false;

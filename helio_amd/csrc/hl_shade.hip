@@ -542,11 +542,10 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     // per-light gradients go to one of kGradSlots copies (by wave) so that the
     // FP64 atomics of many waves on one light do not serialise on one address
     const uint32_t slot = (b * 4u + wave) % kGradSlots;
-    uint32_t ord = 0;
+    OrdinalShare turns{share, part_no};
     walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t li, bool mine) {
-        if ((ord++ & share) != part_no) return;
         adjoint_light(a, L, li, mine, p, gl, cv, ms, slot);
-    });
+    }, nullptr, nullptr, LightShare{}, OneClass{}, &turns);
     float dA[3], dR, dM;
     adjoint_pixel(p, ms, dA, dR, dM);
     // the waves' partial per-pixel gradients, added in wave order
@@ -621,9 +620,9 @@ __device__ __forceinline__ void fused_tile_split(const ShadeArgs& a, uint32_t b,
     KeptLights& kept = as.kept[wave];
     KeptState ks;
     float lo[3] = {0.0f, 0.0f, 0.0f};
-    uint32_t ord = 0;
+    OrdinalShare turns{3u, wave};
     walk_lights<GRID, true>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t, bool mine) {
-        if ((ord++ & 3u) != wave || !mine) return;
+        if (!mine) return;
         Term t;
         if (eval_term<false>(L, p, t)) {
             const float aw = t.atten * t.ndl;
@@ -631,7 +630,7 @@ __device__ __forceinline__ void fused_tile_split(const ShadeArgs& a, uint32_t b,
             lo[1] += t.B[1] * (L.p1.y * aw);
             lo[2] += t.B[2] * (L.p1.z * aw);
         }
-    }, &kept, &ks);
+    }, &kept, &ks, LightShare{}, OneClass{}, &turns);
 #pragma unroll
     for (int c = 0; c < 3; ++c) as.gl[wave][c][lane] = lo[c];
     __syncthreads();
@@ -659,18 +658,17 @@ __device__ __forceinline__ void fused_tile_split(const ShadeArgs& a, uint32_t b,
     const float cv = (1.0f - p.ndv) * hl_f_rcp(p.ev);
     const uint32_t slot = (b * 4u + wave) % kGradSlots;
     if (ks.ok) {
-        for (uint32_t i = wave; i < ks.n; i += 4u) {  // uniform
+        for (uint32_t i = 0; i < ks.n; ++i) {  // uniform
             const HotLight L = s_l[i];
             const uint32_t li = hl_uniform(kept.idx[i]);
             const uint64_t lanes = kept.lanes[i];
             adjoint_light(a, L, li, ((lanes >> lane) & 1ull) != 0ull, p, gl, cv, ms, slot);
         }
     } else {
-        uint32_t ord2 = 0;
+        turns.ord = 0u;
         walk_lights<GRID>(a, s_l, p, valid, cell, [&](const HotLight& L, uint32_t li, bool mine) {
-            if ((ord2++ & 3u) != wave) return;
             adjoint_light(a, L, li, mine, p, gl, cv, ms, slot);
-        });
+        }, nullptr, nullptr, LightShare{}, OneClass{}, &turns);
     }
     float dA[3], dR, dM;
     adjoint_pixel(p, ms, dA, dR, dM);
