@@ -580,9 +580,9 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
 // The fused forward + L2 adjoint of wave tile b & 3 of block tile b >> 2
 // (the items are wave tiles, four per block tile): radiance into a.out, the
 // loss sum((out - target)^2) into a.loss, and its gradients.  The block's
-// four waves share the tile: each walks its lights (keeping the ones it
-// visits in LDS) and evaluates every fourth one (ordinals = wave mod 4) in
-// the forward and the adjoint alike; the waves' partial sums are added in
+// four waves share the tile: each walks its lights and keeps and evaluates
+// every fourth one it finds (ordinals = wave mod 4, records in LDS) in the
+// forward and the adjoint alike; the waves' partial sums are added in
 // wave order, so the output depends on the tile shape at the last bits.
 template <int FA, int FN, int GRID>
 __device__ __forceinline__ void fused_tile_split(const ShadeArgs& a, uint32_t b, ShadeSmem& sm, AdjSmem& as) {
