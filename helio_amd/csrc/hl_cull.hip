@@ -2104,8 +2104,11 @@ __global__ __launch_bounds__(kColThreads) void k_tile_cull(TileArgs a) {
                                  max((int)(r.x >> 16) - (int)ty0, 0), min((int)(r.y >> 16) - (int)ty0, (int)ny - 1));
             }
             *reinterpret_cast<uint64_t*>(sm.tiles[t]) = mask;
-            if (t == 0u) sm.open[(batch + 1u) & 1u] = 0u;  // read last before the previous barrier
             __syncthreads();
+            // the next batch's flag: every wave's read of it for the previous
+            // batch is before this barrier, the next batch's adds are after
+            // the one below
+            if (t == 0u) sm.open[(batch + 1u) & 1u] = 0u;
             // the wave's row of tiles
             bool some = false;
             if (wave < ny) {
