@@ -351,7 +351,7 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     constexpr bool kShared = MODE == kModeForward && DIV == kShare;
     constexpr bool split = kAdj || kShared;
     [[maybe_unused]] const bool classes =
-        MODE == kModeForward && DIV == kClasses && forward_split(a.width, a.height, a.num_lights);
+        MODE == kModeForward && DIV == kClasses && forward_split(GRID, a.width, a.height, a.num_lights);
     const uint32_t twl = a.tw_log2, tw = 1u << twl;
     const uint32_t th = 64u >> twl;
     // 2^sh waves share a tile; this one is number part_no of them, and the block
@@ -1077,7 +1077,7 @@ static hipError_t launch_fmt(hipStream_t s, int set, const ShadeArgs& a, uint32_
 hipError_t launch_shade(hipStream_t s, int gbuf_set, int mode, const ShadeArgs& a, uint32_t* queue,
                         uint32_t* queue_next) {
     if (a.num_blocks == 0) return hipSuccess;
-    if (mode == kModeForward && forward_split(a.width, a.height, a.num_lights))
+    if (mode == kModeForward && forward_split((uint32_t)a.grid_mode, a.width, a.height, a.num_lights))
         return a.out_f16 ? launch_fmt<kModeForward | kModeShared | kModeOutF16>(s, gbuf_set, a, queue, queue_next)
                          : launch_fmt<kModeForward | kModeShared>(s, gbuf_set, a, queue, queue_next);
     if (a.out_f16) {  // the modes that write the radiance alone take an RGBA16F target

@@ -1,0 +1,31 @@
+"""Which launches the host code takes for a call (CPU only, hip_routes)."""
+import pytest
+
+from hip_routes import routes
+
+SHARED = 16  # kModeShared: four waves to a wave tile
+
+
+def test_forward_shares_wave_tiles_only_where_that_is_faster():
+    """Sharing repeats a tile's set-up and walk four times: sizes and light counts on both sides of where the
+    two forms took the same time, on clusters and on tile lists (which end at 64 lights)."""
+    cases = [  # width, height, lights, shared on clusters, on tiles
+        (64, 64, 4, False, False), (32, 32, 15, False, False), (64, 64, 16, True, True),
+        (128, 128, 31, False, False), (128, 128, 64, True, True), (256, 256, 64, False, False),
+        (256, 256, 128, True, True), (333, 177, 16, False, False), (352, 352, 512, True, True),
+        (512, 512, 256, False, False), (512, 512, 512, True, False), (720, 720, 1024, False, False),
+        (720, 720, 4096, True, False), (1024, 1024, 749, False, False), (1024, 1024, 16384, False, False),
+    ]
+    got = routes(f"""
+for w, h, n, _, _ in {cases!r}:
+    row = []
+    for grid in ((4, 4, 24), None):
+        ds, cull = cull_pass(scene(n, w, h), grid)
+        sh = DeferredLightPass(ctx, w, h)
+        sh.prepare(ds)
+        mode = [v[3] for k, v, _ in calls(lambda: sh.execute(ds, cull.publish())) if k == "k_shade"]
+        row.append(mode == [{SHARED}])
+    result.append(row)
+""")
+    for c, g in zip(cases, got):
+        assert g == list(c[3:]), c
