@@ -92,6 +92,7 @@ struct hl_plan {
     // launch per non-empty group; group = set * 2 + (adjoint ? 1 : 0)
     uint32_t grp_first[6] = {}, grp_spans[6] = {}, grp_count[6] = {}, grp_grid[6] = {};
     uint32_t grp_view[6] = {};  // the view of a group of one view
+    int grp_mode[6] = {};       // of its launch: kModeShared with a view that forward_split holds for
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -181,7 +182,7 @@ hl_status enqueue_frame(hl_plan* p, hipStream_t s) {
     const hl_status cs = enqueue_cull(p, s);
     if (cs != HL_OK) return cs;
     for (int g = 0; g < 6; ++g)
-        HL_HIP(c, launch_shade_batch(s, g / 2, (g & 1) ? kModeFusedL2 : kModeForward, p->d_shade,
+        HL_HIP(c, launch_shade_batch(s, g / 2, p->grp_mode[g], p->d_shade,
                                      p->d_spans + p->grp_first[g], p->grp_spans[g], p->grp_count[g],
                                      p->d_queue + (size_t)g * kShadeQueueWords, p->grp_grid[g],
                                      p->grp_spans[g] == 1u ? &p->hshade[p->grp_view[g]].sa : nullptr));
@@ -395,12 +396,16 @@ hl_status build_plan(hl_plan* p) {
     uint64_t all_items = 0;
     for (int g = 0; g < 6; ++g) {
         p->grp_first[g] = (uint32_t)spans.size();
+        p->grp_mode[g] = (g & 1) ? kModeFusedL2 : kModeForward;
         uint64_t n = 0;
         for (const auto& o : order) {
             const uint32_t v = o.second;
             if (vset[v] * 2 + (is_adjoint(p->views[v]) ? 1 : 0) != g) continue;
             spans.push_back(make_uint2((uint32_t)n, v));
             p->grp_view[g] = v;
+            const ShadeArgs& a = p->hshade[v].sa;
+            if (!(g & 1) && forward_split(a.grid_mode, a.width, a.height, a.num_lights))
+                p->grp_mode[g] = kModeForward | kModeShared;
             n += is_adjoint(p->views[v]) ? shade_items<kModeFusedL2>(p->hshade[v].sa)
                                           : shade_items<kModeForward>(p->hshade[v].sa);
         }
@@ -410,8 +415,7 @@ hl_status build_plan(hl_plan* p) {
         p->grp_count[g] = (uint32_t)n;
         all_items += n;
         // the blocks the kernel keeps resident, fewer when there are fewer items
-        p->grp_grid[g] = std::min((uint32_t)std::max(1, cus) * shade_batch_blocks_per_cu(g / 2, (g & 1) ? kModeFusedL2
-                                                                                                    : kModeForward),
+        p->grp_grid[g] = std::min((uint32_t)std::max(1, cus) * shade_batch_blocks_per_cu(g / 2, p->grp_mode[g]),
                                   std::max(1u, p->grp_count[g]));
     }
     p->num_items = (uint32_t)all_items;

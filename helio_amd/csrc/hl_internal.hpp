@@ -227,7 +227,8 @@ enum ShadeMode : int {
     // flag on the forward-writing modes (forward, shadowed, extended): the
     // output target is RGBA16F (ShadeArgs::out_f16) instead of RGBA32F
     kModeOutF16 = 8,
-    // flag on kModeForward: the view's wave tiles are shared (forward_split)
+    // flag on kModeForward: the view's wave tiles are shared (forward_split); a
+    // batched launch holds such a view
     kModeShared = 16
 };
 constexpr int kModeMask = 7;
@@ -341,6 +342,8 @@ hipError_t launch_forward_prep(hipStream_t s, const GpuLight* lights, uint32_t n
                                const hl_transform* transforms, uint32_t num_transforms, HotLight* hot);
 hipError_t launch_forward_lit(hipStream_t s, const ForwardArgs& a);
 
+// mode: kModeForward, kModeForward | kModeShared (forward_split holds for a view)
+// or kModeFusedL2.
 // spans: nspans (first item, view) pairs in item order, then (num_items, 0).
 // queue: kShadeQueueWords claim counters, zero before the first launch; each
 // launch leaves them zero (its last block out clears them).  one: the

@@ -325,9 +325,9 @@ __device__ __forceinline__ void adjoint_light(const ShadeArgs& a, const HotLight
 // How the forward mode divides a view that forward_split holds for.  kOwn: the
 // view is not one; a wave has its own tile and one sum.  kShare: the block's
 // four waves share a tile, each the lights of one index modulo 4.  kClasses
-// (batched launches, which have waves enough and cannot choose per view at
-// compile time): a wave has its own tile and keeps the four sums apart on
-// such a view, so that the pixel is kShare's bit for bit.
+// (batched launches that hold such a view; they have waves enough): a wave has
+// its own tile and keeps the four sums apart on such a view, so that the pixel
+// is kShare's bit for bit.
 enum LightDivision : int { kOwn = 0, kShare = 1, kClasses = 2 };
 
 // Every mode but the fused forward + adjoint (fused_tile).
@@ -351,7 +351,7 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a, uint32_t b, Shade
     constexpr bool kShared = MODE == kModeForward && DIV == kShare;
     constexpr bool split = kAdj || kShared;
     [[maybe_unused]] const bool classes =
-        MODE == kModeForward && DIV == kClasses && forward_split(GRID, a.width, a.height, a.num_lights);
+        DIV == kClasses && forward_split(GRID, a.width, a.height, a.num_lights);
     const uint32_t twl = a.tw_log2, tw = 1u << twl;
     const uint32_t th = 64u >> twl;
     // 2^sh waves share a tile; this one is number part_no of them, and the block
@@ -895,7 +895,12 @@ __global__ __launch_bounds__(256, (shade_min_blocks<(MODE & kModeMask), FA>())) 
 // (first item, view); an item's view and tile follow from its index.  One
 // launch covers the views of one G-buffer format set and one mode (forward,
 // or forward + L2 adjoint): the adjoint needs about twice the registers,
-// which would halve the forward's occupancy in a shared kernel.  A block
+// which would halve the forward's occupancy in a shared kernel.  A forward
+// launch has the class sums (kModeShared) only when one of its views needs them:
+// their 9 KB of LDS and a test and a ballot per light class cost the others 1 to
+// 3 % (frames of one 4K view with 1024 lights 184.3 -> 179.3 us without, of two
+// 1080p views 118.6 -> 116.5); two launches for a plan that holds both kinds cost
+// more, the first one's tail (a 720p view and two faces 57 -> 68 us).  A block
 // keeps the item range of its current view; when an item falls outside it
 // (rare: each sub-queue's items run through one view at a time) the block
 // finds the span by bisection and stages that view's constants in LDS.  The
@@ -910,18 +915,20 @@ typedef const __attribute__((address_space(4))) BatchShadeView* ConstViews;
 // arguments the tile uses in its loops were reloaded there (18x the scalar
 // loads of k_shade on the same tiles) rather than kept in scalar registers.
 template <int FA, int FN, int MODE>
-__global__ __launch_bounds__(256, MODE == kModeForward ? 5 : 1) void k_shade_batch(
+__global__ __launch_bounds__(256, (MODE & kModeMask) == kModeForward ? 5 : 1) void k_shade_batch(
     ConstViews __restrict__ views, const uint2* __restrict__ spans, uint32_t nspans,
     uint32_t num_items, uint32_t* __restrict__ queue, ShadeArgs one) {
+    constexpr int M = MODE & kModeMask;
+    constexpr LightDivision kDiv = (MODE & kModeShared) ? kClasses : kOwn;
     __shared__ ShadeSmem sm;
     __shared__ ClaimSmem cs;
     AdjSmem* as = nullptr;
-    if constexpr (MODE == kModeFusedL2) {
+    if constexpr (M == kModeFusedL2) {
         __shared__ AdjSmem adj;
         as = &adj;
     }
     ClassSmem* cl = nullptr;
-    if constexpr (MODE == kModeForward) {
+    if constexpr (kDiv == kClasses) {
         __shared__ ClassSmem classes;
         cl = &classes;
     }
@@ -929,8 +936,8 @@ __global__ __launch_bounds__(256, MODE == kModeForward ? 5 : 1) void k_shade_bat
     if (nspans == 1u) {
         load_view_const(one, sm);  // published by the first claim's barrier
         claim_items(num_items, queue, cs, [&](uint32_t it) {
-            if constexpr (MODE == kModeFusedL2) fused_tile<FA, FN, HL_GRID_CLUSTERS>(one, it, sm, *as);
-            else shade_tile<FA, FN, HL_GRID_CLUSTERS, MODE, false, kClasses>(one, it, sm, as, cl);
+            if constexpr (M == kModeFusedL2) fused_tile<FA, FN, HL_GRID_CLUSTERS>(one, it, sm, *as);
+            else shade_tile<FA, FN, HL_GRID_CLUSTERS, M, false, kDiv>(one, it, sm, as, cl);
         });
     } else claim_items(num_items, queue, cs, [&](uint32_t it) {
         it = hl_uniform(it);  // block-uniform: every thread read the same claim
@@ -951,8 +958,8 @@ __global__ __launch_bounds__(256, MODE == kModeForward ? 5 : 1) void k_shade_bat
         // v again as a scalar: carried across the claim loop it is not known
         // to be uniform
         const ShadeArgs& ra = *(const ShadeArgs*)&views[hl_uniform(v)].sa;
-        if constexpr (MODE == kModeFusedL2) fused_tile<FA, FN, HL_GRID_CLUSTERS>(ra, it - first, sm, *as);
-        else shade_tile<FA, FN, HL_GRID_CLUSTERS, MODE, false, kClasses>(ra, it - first, sm, as, cl);
+        if constexpr (M == kModeFusedL2) fused_tile<FA, FN, HL_GRID_CLUSTERS>(ra, it - first, sm, *as);
+        else shade_tile<FA, FN, HL_GRID_CLUSTERS, M, false, kDiv>(ra, it - first, sm, as, cl);
     });
     // The last block out clears the claim counters for the next launch, so a
     // captured graph replays this launch unchanged.  Blocks that have finished
@@ -984,9 +991,13 @@ template <int FA, int FN>
 static void launch_batch_fmt(hipStream_t s, int mode, const BatchShadeView* views, const uint2* spans,
                              uint32_t nspans, uint32_t num_items, uint32_t* queue, uint32_t grid_blocks,
                              const ShadeArgs& one) {
+    constexpr int kClassed = kModeForward | kModeShared;
     if (mode == kModeFusedL2)
         k_shade_batch<FA, FN, kModeFusedL2><<<grid_blocks, 256, 0, s>>>((ConstViews)views, spans, nspans, num_items,
                                                                         queue, one);
+    else if (mode == kClassed)
+        k_shade_batch<FA, FN, kClassed><<<grid_blocks, 256, 0, s>>>((ConstViews)views, spans, nspans, num_items,
+                                                                    queue, one);
     else
         k_shade_batch<FA, FN, kModeForward><<<grid_blocks, 256, 0, s>>>((ConstViews)views, spans, nspans, num_items,
                                                                         queue, one);
@@ -994,10 +1005,12 @@ static void launch_batch_fmt(hipStream_t s, int mode, const BatchShadeView* view
 
 template <int FA, int FN>
 static uint32_t batch_blocks_per_cu(int mode) {
+    constexpr int kClassed = kModeForward | kModeShared;
+    const auto kernel = mode == kModeFusedL2 ? k_shade_batch<FA, FN, kModeFusedL2>
+                        : mode == kClassed   ? k_shade_batch<FA, FN, kClassed>
+                                             : k_shade_batch<FA, FN, kModeForward>;
     int n = 0;
-    const hipError_t e = mode == kModeFusedL2
-                             ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_shade_batch<FA, FN, kModeFusedL2>, 256, 0)
-                             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_shade_batch<FA, FN, kModeForward>, 256, 0);
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 256, 0);
     return e == hipSuccess && n > 0 ? (uint32_t)n : 1u;
 }
 

@@ -29,3 +29,23 @@ for w, h, n, _, _ in {cases!r}:
 """)
     for c, g in zip(cases, got):
         assert g == list(c[3:]), c
+
+
+def test_batched_launch_has_class_sums_only_for_a_view_that_needs_them():
+    """The class sums of shared wave tiles cost LDS, a test and a ballot per light class: plans without a shared
+    view do not pay for them; a plan with one still has one forward launch."""
+    own, shared = (1, 2, 0), (1, 2, SHARED)
+    plans = [([(512, 288, 64)], [own]), ([(640, 360, 100)] * 3, [own]), ([(128, 128, 256)] * 2, [shared]),
+             ([(512, 288, 64), (128, 128, 256), (128, 128, 256)], [shared])]
+    got = routes(f"""
+for views, _ in {plans!r}:
+    made = []
+    for w, h, n in views:
+        sc = scene(n, w, h)
+        made.append(BatchView(scene=upload_scene(ctx, sc), subset=ctx.upload(np.arange(n, dtype=np.uint32)),
+                              num_lights=n, out=ctx.alloc(w * h * 16)))
+    plan = BatchPlan(ctx, made[-1].scene.lights, views[-1][2], made)
+    result.append([v for k, v, _ in calls(plan.launch) if k == "k_shade_batch"])
+""")
+    for (views, want), g in zip(plans, got):
+        assert [tuple(v) for v in g] == want, views
