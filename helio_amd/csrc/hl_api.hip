@@ -621,10 +621,11 @@ HL_API hl_status hl_light_cull_clusters(hl_context* c, const GpuCameraUniforms* 
     if ((s = ensure(c, c->cull, sizeof(CullLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
     if ((s = ensure(c, c->hot, sizeof(HotLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
     if ((s = ensure(c, c->raw, cluster_raw_bytes((uint32_t)ncell))) != HL_OK) return s;
-    const size_t columns = column_scratch_bytes(p->grid_x, p->grid_y, p->grid_z, n);
-    if (columns) {
-        if ((s = ensure(c, c->columns, columns)) != HL_OK) return s;
-    } else {
+    const ClusterPath path = cluster_path(p->grid_x, p->grid_y, p->grid_z, n);
+    if (path == ClusterPath::kColumns) {
+        s = ensure(c, c->columns, column_scratch_bytes(p->grid_x, p->grid_y, p->grid_z, n));
+        if (s != HL_OK) return s;
+    } else if (path == ClusterPath::kMark) {
         if ((s = ensure(c, c->geom, cluster_geom_bytes(ncol, (uint32_t)ncell))) != HL_OK) return s;
         if ((s = ensure(c, c->bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
         if ((s = ensure(c, c->summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;
@@ -639,7 +640,7 @@ HL_API hl_status hl_light_cull_clusters(hl_context* c, const GpuCameraUniforms* 
     ClusterScratch w{c->geom.p, (uint32_t*)c->bits.p, (uint32_t*)c->summary.p, (uint32_t*)c->raw.p,
                      mark_queue_at(c->markq.p, n), c->columns.p};
     HL_HIP(c, launch_cluster_cull(c->stream, a, camera_d, lights_d, (HotLight*)c->hot.p, (CullLight*)c->cull.p,
-                                  ctx_words(c) + 1, w, offsets_d, counts_d, pool_d, pool_cap, flags, flags2));
+                                  ctx_words(c) + 1, path, w, offsets_d, counts_d, pool_d, pool_cap, flags, flags2));
     c->hot_src = lights_d;
     c->hot_n = n;
     return HL_OK;

@@ -24,6 +24,8 @@
 //                     bitmask, which it clears again for the next call
 //  k_col_*            the clustered lists a column of the grid per block (most
 //                     grids; see the section)
+//  k_cluster_bf_*     the clustered lists by testing every light in every cell
+//                     (small problems on wide grids of few slices)
 //  k_batch_*          the same steps for many views in one launch each
 // Membership is decided by the same exact FP32 tests whatever the order of
 // evaluation, so the lists equal the per-cluster brute force bit for bit.
@@ -904,8 +906,155 @@ __device__ __forceinline__ CellBox* view_boxes(const BatchCullView& v) {
     return (CellBox*)((uint8_t*)v.geom + cluster_geom_offset_boxes_dev(v.ca.grid_x * v.ca.grid_y));
 }
 
+// ------------------------------------------------- clusters, brute force
+// Two launches for small problems (cells x lights <= kSmallTests) on wide grids
+// of few slices (cluster_path): every cell tests every light with the
+// membership rule (cell_member), one wave per cell and four cells per block,
+// the lights' culling records built per block into LDS kBfLights at a time,
+// each cell's records built by its own wave in registers.  k_cluster_bf_count
+// stores each cell's member count (and the lights' shading records);
+// k_cluster_bf_fill finds each cell's offset from the capped counts before
+// it, then writes the ascending list.  Membership does not depend on the
+// order of evaluation, so the lists are the other paths'.
+constexpr uint64_t kSmallTests = 1ull << 22;
+constexpr uint32_t kBfCells = 4;  // one per wave
+constexpr uint32_t kBfLights = 256;
+
+struct BfSmem {
+    CullLight light[kBfLights];
+    uint32_t capped[kBfCells];
+    unsigned long long part[4];
+    uint32_t flags;
+};
+
+// The records of the wave's cell (every lane alike).
+struct BfCell {
+    ColumnGeom g;
+    CellBox bx;
+    float pad;
+};
+__device__ __forceinline__ BfCell bf_cell(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
+                                          uint32_t cell, uint32_t ncell) {
+    BfCell c;
+    const uint32_t ncol = a.grid_x * a.grid_y;
+    if (cell < ncell) {
+        cell_geometry(a, cam, cell % ncol, cell / ncol, true, c.g, c.bx);
+        c.pad = a.slice_r_pad[cell / ncol];
+    } else {  // no cell: no member (the records are not read)
+        c.g = ColumnGeom{};
+        c.bx = CellBox{};
+        c.pad = 0.0f;
+    }
+    return c;
+}
+
+// For each light of the LDS chunk [l0, l0 + kBfLights) in ascending order, in
+// groups of 64: f(group, pass) with pass this lane's light's membership in
+// the wave's cell (uniform calls).
+template <class F>
+__device__ __forceinline__ void bf_chunk(const ClusterArgs& a, uint32_t l0, const BfCell& c, const BfSmem& sm,
+                                         F&& f) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t nl = a.num_lights - l0 < kBfLights ? a.num_lights - l0 : kBfLights;
+    for (uint32_t j0 = 0; j0 < nl; j0 += 64u) {
+        const uint32_t j = j0 + lane;
+        const bool pass = c.g.on != 0u && j < nl && cell_member(sm.light[j], c.g, c.bx, c.pad);
+        f(j0, pass);
+    }
+}
+
+__device__ __forceinline__ void bf_load_lights(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
+                                               const GpuLight* __restrict__ lights, uint32_t l0, BfSmem& sm) {
+    __syncthreads();  // the previous chunk is no longer read
+    const uint32_t i = l0 + threadIdx.x;
+    if (i < a.num_lights) sm.light[threadIdx.x] = cull_light_at(lights, i, cam);
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void k_cluster_bf_count(ClusterArgs a, const GpuCameraUniforms* __restrict__ cam,
+                                                          const GpuLight* __restrict__ lights,
+                                                          HotLight* __restrict__ hot,
+                                                          uint32_t* __restrict__ feature_flags,
+                                                          uint32_t* __restrict__ raw, uint32_t* __restrict__ flags,
+                                                          uint32_t* __restrict__ flags2) {
+    __shared__ BfSmem sm;
+    const uint32_t ncell = a.grid_x * a.grid_y * a.grid_z;
+    const uint32_t cell = blockIdx.x * kBfCells + (threadIdx.x >> 6);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // OR-ed by the fill launch
+        *flags = 0u;
+        if (flags2) *flags2 = 0u;
+    }
+    // the shading records, grid-stride over the lights
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.num_lights; i += gridDim.x * blockDim.x)
+        prep_one(lights, nullptr, a.num_lights, cam, hot, nullptr, feature_flags, i);
+    const BfCell c = bf_cell(a, cam, cell, ncell);
+    uint32_t cnt = 0u;
+    for (uint32_t l0 = 0; l0 < a.num_lights; l0 += kBfLights) {
+        bf_load_lights(a, cam, lights, l0, sm);
+        bf_chunk(a, l0, c, sm, [&](uint32_t, bool pass) { cnt += (uint32_t)__popcll(hl_ballot(pass)); });
+    }
+    if ((threadIdx.x & 63u) == 0 && cell < ncell) raw[cell] = cnt;
+}
+
+__global__ __launch_bounds__(256) void k_cluster_bf_fill(ClusterArgs a, const GpuCameraUniforms* __restrict__ cam,
+                                                         const GpuLight* __restrict__ lights,
+                                                         const uint32_t* __restrict__ raw, uint32_t pool_cap,
+                                                         uint32_t* __restrict__ offsets, uint32_t* __restrict__ counts,
+                                                         uint32_t* __restrict__ pool, uint32_t* __restrict__ flags,
+                                                         uint32_t* __restrict__ flags2) {
+    __shared__ BfSmem sm;
+    const uint32_t ncell = a.grid_x * a.grid_y * a.grid_z, first = blockIdx.x * kBfCells;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    const uint32_t cell = first + wave, cap = a.cap;
+    // capped counts of the cells before the block
+    unsigned long long acc = 0;
+    for (uint32_t j = t; j < first; j += blockDim.x) {
+        const uint32_t v = raw[j];
+        acc += (cap && v > cap) ? cap : v;
+    }
+    acc = wave_sum_u64(acc);
+    if (lane == 0) sm.part[wave] = acc;
+    if (t == 0) sm.flags = 0u;
+    if (t < kBfCells) {
+        const uint32_t v = first + t < ncell ? raw[first + t] : 0u;
+        sm.capped[t] = (cap && v > cap) ? cap : v;
+    }
+    const BfCell c = bf_cell(a, cam, cell, ncell);
+    __syncthreads();
+    // the wave's cell: offset, count after the cap and the pool truncation
+    unsigned long long base = sm.part[0] + sm.part[1] + sm.part[2] + sm.part[3];
+    for (uint32_t j = 0; j < wave; ++j) base += sm.capped[j];
+    const uint32_t o = base > pool_cap ? pool_cap : (uint32_t)base;
+    uint32_t cnt = sm.capped[wave], fl = 0u;
+    if (cell < ncell && cap && raw[cell] > cap) fl |= HL_OVERFLOW_CAP;
+    if (cnt > pool_cap - o) {
+        cnt = pool_cap - o;
+        fl |= HL_OVERFLOW_POOL;
+    }
+    if (lane == 0 && cell < ncell) {
+        offsets[cell] = o;
+        counts[cell] = cnt;
+        if (fl) atomicOr(&sm.flags, fl);
+    }
+    uint32_t written = 0u;
+    for (uint32_t l0 = 0; l0 < a.num_lights; l0 += kBfLights) {
+        bf_load_lights(a, cam, lights, l0, sm);
+        bf_chunk(a, l0, c, sm, [&](uint32_t j0, bool pass) {
+            const uint64_t m = hl_ballot(pass);
+            const uint32_t pos = written + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            if (pass && pos < cnt) pool[o + pos] = l0 + j0 + lane;
+            written += (uint32_t)__popcll(m);
+        });
+    }
+    __syncthreads();
+    if (t == 0 && sm.flags) {
+        atomicOr(flags, sm.flags);
+        if (flags2) atomicOr(flags2, sm.flags);
+    }
+}
+
 // --------------------------------------------- clusters, column by column
-// The path of every grid that use_columns accepts.  A block owns one column of
+// The path of most grids (cluster_path).  A block owns one column of
 // the grid, or kb slices of it when there are few columns (column_plan aims at
 // kColBlocks blocks, two to three per CU):
 //   k_col_prep   one thread per light: its shading and culling records and
@@ -942,9 +1091,9 @@ constexpr uint32_t kColBatch = 512;    // candidates a fill block lists at a tim
 constexpr uint32_t kColGroup = 16;     // columns per partial sum of counts
 
 // A light's candidate cells (inclusive ranges).  col: its columns, a byte each
-// for x0, y0, 127 - x1 and 127 - y1 (grids of at most 128 columns a side), so
-// that one subtraction holds a column against all four ends; slice: s0 | s1 << 8,
-// the top bit set for a light with a cone test.
+// for x0, y0, 127 - x1 and 127 - y1 (in columns >> shift, at most 128 a side),
+// so that one subtraction holds a column against all four ends; slice: s0 |
+// s1 << 8, the top bit set for a light with a cone test.
 struct LightBox {
     uint32_t col, slice;
 };
@@ -954,7 +1103,7 @@ constexpr uint32_t kColMaxSide = 128;
 __device__ __forceinline__ uint32_t box_s0(uint32_t s) { return s & 0xFFu; }
 __device__ __forceinline__ uint32_t box_s1(uint32_t s) { return (s >> 8) & 0xFFu; }
 
-// Sums of counts fit in 32 bits: use_columns keeps cells x lights at 2^31.
+// Sums of counts fit in 32 bits: cluster_path keeps cells x lights at 2^31.
 struct ColumnArgs {
     const GpuCameraUniforms* cam;
     const GpuLight* lights;
@@ -974,6 +1123,7 @@ struct ColumnArgs {
     uint32_t* pool;
     uint32_t pool_cap;
     uint32_t kb;              // slices per block
+    uint32_t shift;           // of the columns in box_col
     uint32_t* flags;
     uint32_t* flags2;
 };
@@ -1007,7 +1157,7 @@ __device__ __forceinline__ int count_below(const float* v, int n, float x) {
 
 // light_cells for one thread, the slice limits by bisection.
 __device__ __forceinline__ LightBox light_box(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
-                                           float4 vpos, bool cone, const SliceTab& t) {
+                                             float4 vpos, bool cone, const SliceTab& t, uint32_t shift) {
     const int gx = (int)a.grid_x, gy = (int)a.grid_y, gz = (int)a.grid_z;
     int x0 = 0, x1 = gx - 1, y0 = 0, y1 = gy - 1, s0 = 0, s1 = gz - 1;
     const LightBox none{kNoBox, 0u};
@@ -1032,7 +1182,9 @@ __device__ __forceinline__ LightBox light_box(const ClusterArgs& a, const GpuCam
     s0 = clampi(s0, 0, gz - 1);
     s1 = clampi(s1, -1, gz - 1);
     if (x1 < x0 || y1 < y0 || s1 < s0) return none;
-    return LightBox{(uint32_t)x0 | (uint32_t)y0 << 8 | (uint32_t)(127 - x1) << 16 | (uint32_t)(127 - y1) << 24,
+    const uint32_t bx0 = (uint32_t)x0 >> shift, by0 = (uint32_t)y0 >> shift;
+    const uint32_t bx1 = (uint32_t)x1 >> shift, by1 = (uint32_t)y1 >> shift;
+    return LightBox{bx0 | by0 << 8 | (127u - bx1) << 16 | (127u - by1) << 24,
                     (uint32_t)s0 | (uint32_t)s1 << 8 | (cone ? kBoxCone : 0u)};
 }
 
@@ -1252,7 +1404,7 @@ __device__ __forceinline__ void col_prep_block(const ClusterArgs& a, const Colum
     }
     const CullLight L = cull_light_at(p.lights, p.subset ? p.subset[i] : i, p.cam);
     p.cull[i] = L;
-    const LightBox b = light_box(a, p.cam, L.vpos, L.cone.w != kNoCone, tab);
+    const LightBox b = light_box(a, p.cam, L.vpos, L.cone.w != kNoCone, tab, p.shift);
     p.box_col[i] = b.col;
     p.box_slice[i] = b.slice;
     prep_one(p.lights, p.subset, a.num_lights, p.cam, p.hot, nullptr, p.feature_flags, i);
@@ -1285,7 +1437,7 @@ __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const Colu
         __syncthreads();
     }
     const bool on = col_setup(a, p.cam, c, sm.g);
-    const uint32_t key = column_key(c.cx, c.cy), k1 = c.k0 + c.nk - 1u;
+    const uint32_t key = column_key(c.cx >> p.shift, c.cy >> p.shift), k1 = c.k0 + c.nk - 1u;
     [[maybe_unused]] const bool part_column = c.nk != a.grid_z;
     if (INLINE && block == 0 && t == 0) {
         *p.flags = 0u;
@@ -1306,7 +1458,7 @@ __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const Colu
                                               hl_x_mat_row(v, 1, pr.x, pr.y, pr.z, 1.0f),
                                               hl_x_mat_row(v, 2, pr.x, pr.y, pr.z, 1.0f),
                                               type == HL_LIGHT_DIRECTIONAL ? __builtin_inff() : pr.w);
-                const LightBox b = light_box(a, p.cam, vp, type == HL_LIGHT_SPOT, sm.g.tab);
+                const LightBox b = light_box(a, p.cam, vp, type == HL_LIGHT_SPOT, sm.g.tab, p.shift);
                 inline_slices[t] = b.slice;
                 m = on && box_has_column(b.col, key) && box_has_slices(b.slice, c.k0, k1);
             }
@@ -1551,7 +1703,26 @@ static ColumnPlan column_plan(uint32_t ncol, uint32_t gz, uint32_t aim) {
 // a side) and 2^25 (block, light) pairs.
 static bool use_columns(uint32_t gx, uint32_t gy, uint32_t gz, uint64_t n) {
     const uint32_t ncol = gx * gy;
-    return gx <= kColMaxSide && gy <= kColMaxSide && ncol <= kColMaxColumns && column_plan(ncol, gz, kColBlocks).blocks * n <= (1ull << 25);
+    return gx <= kColMaxSide && gy <= kColMaxSide && ncol <= kColMaxColumns &&
+           column_plan(ncol, gz, kColBlocks).blocks * n <= (1ull << 25);
+}
+// Small problems of a single view on wider grids: the brute force where a
+// column is only a cell or a few (up to 65536 cells: its fill reads every count
+// before its own), else the column path (the lights' boxes in coarser columns);
+// the mark path's two atomics per member make it the slowest where lights are
+// large, though the fastest where they are small.  Calls, us, brute force /
+// columns / mark path with the lights of a scene, and with every light in every
+// cell: 256x144x1 cells and 100 lights 144 / 368 / 294, 136 / 447 / 450; 80x45x1
+// and 1000 47 / 55 / 79, 43 / 106 / 119; 160x90x1 and 290 71 / 153 / 166, 82 /
+// 299 / 217; 128x72x4 and 100 143 / 89 / 31, 135 / 155 / 490; 64x36x8 and 200
+// 78 / 35 / 29, 71 / 73 / 288; 80x45x24 and 48 414 / 55 / 36, 407 / 134 / 1020;
+// 200x1x1 and 5000 115 / 31 / 56, 86 / 41 / 130.
+ClusterPath cluster_path(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n) {
+    const uint32_t ncol = gx * gy;
+    const uint64_t ncell = (uint64_t)ncol * gz;
+    if (use_columns(gx, gy, gz, n)) return ClusterPath::kColumns;
+    if (ncell * n > kSmallTests) return ClusterPath::kMark;
+    return gz < 4u && ncol > kColBlocks && ncell <= 65536u ? ClusterPath::kBruteForce : ClusterPath::kColumns;
 }
 static bool column_inline(uint32_t ncell, uint32_t n) { return n <= kColInline && ncell <= kColInlineCells; }
 
@@ -1582,7 +1753,6 @@ static size_t column_scratch(uint8_t* base, uint32_t ncol, uint32_t gz, uint32_t
 }
 size_t column_scratch_bytes(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n) {
     const uint32_t ncol = gx * gy;
-    if (!use_columns(gx, gy, gz, n)) return 0;
     return column_scratch(nullptr, ncol, gz, n, column_plan(ncol, gz, kColBlocks).blocks, nullptr);
 }
 
@@ -2247,12 +2417,21 @@ size_t cluster_geom_bytes(uint32_t ncol, uint32_t ncell) {
 
 hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCameraUniforms* cam,
                                const GpuLight* lights, HotLight* hot, CullLight* cl, uint32_t* feature_flags,
-                               const ClusterScratch& w, uint32_t* offsets,
+                               ClusterPath path, const ClusterScratch& w, uint32_t* offsets,
                                uint32_t* counts, uint32_t* pool, uint32_t pool_cap,
                                uint32_t* flags, uint32_t* flags2) {
     const uint32_t ncol = a.grid_x * a.grid_y;
     const uint32_t ncell = ncol * a.grid_z;
-    if (use_columns(a.grid_x, a.grid_y, a.grid_z, a.num_lights)) {
+    if (path == ClusterPath::kBruteForce) {
+        const uint32_t blocks = (ncell + kBfCells - 1u) / kBfCells;
+        k_cluster_bf_count<<<blocks, 256, 0, s>>>(a, cam, lights, hot, feature_flags, w.raw, flags, flags2);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        k_cluster_bf_fill<<<blocks, 256, 0, s>>>(a, cam, lights, w.raw, pool_cap, offsets, counts, pool, flags,
+                                                 flags2);
+        return hipGetLastError();
+    }
+    if (path == ClusterPath::kColumns) {
         const ColumnPlan cp = column_plan(ncol, a.grid_z, kColBlocks);
         ColumnArgs p{};
         p.cam = cam;
@@ -2266,6 +2445,7 @@ hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCam
         p.pool = pool;
         p.pool_cap = pool_cap;
         p.kb = cp.kb;
+        while ((std::max(a.grid_x, a.grid_y) - 1u) >> p.shift >= kColMaxSide) ++p.shift;
         p.flags = flags;
         p.flags2 = flags2;
         (void)column_scratch((uint8_t*)w.columns, ncol, a.grid_z, a.num_lights, cp.blocks, &p);
@@ -2279,7 +2459,10 @@ hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCam
         k_col_prep<<<a.num_lights ? (a.num_lights + 63u) / 64u : 1u, 64, 0, s>>>(
             a, p, column_groups(ncol) * a.grid_z);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        k_col_count<kColChunk, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+        if (ncol <= kColMaxColumns)
+            k_col_count<kColChunk, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+        else  // many small blocks: the smaller list lets four share a CU
+            k_col_count<kBatchColChunk, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         k_col_fill<true><<<cp.blocks, 256, 0, s>>>(a, p);
         return hipGetLastError();

@@ -140,8 +140,10 @@ struct ClusterScratch {
     MarkQueue mq;        // mark_queue_bytes(lights)
     void* columns;       // column_scratch_bytes(columns, slices, lights)
 };
-// Scratch of the column path of the clustered cull; 0: the grid and the lights
-// take the mark path (which alone needs geom, bits, summary and mq).
+// How a single view's clusters are built.  Every path needs raw; the mark path
+// geom, bits, summary and mq, the column path columns.
+enum class ClusterPath { kColumns, kBruteForce, kMark };
+ClusterPath cluster_path(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t num_lights);
 size_t column_scratch_bytes(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t num_lights);
 size_t cluster_geom_bytes(uint32_t ncol, uint32_t ncell);
 size_t cluster_geom_offset_boxes(uint32_t ncol);
@@ -208,7 +210,7 @@ hipError_t launch_batch_columns(hipStream_t s, const void* views, const uint32_t
 // flags) and builds the lists.
 hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCameraUniforms* cam,
                                const GpuLight* lights, HotLight* hot, CullLight* cl, uint32_t* feature_flags,
-                               const ClusterScratch& w, uint32_t* offsets,
+                               ClusterPath path, const ClusterScratch& w, uint32_t* offsets,
                                uint32_t* counts, uint32_t* pool, uint32_t pool_cap,
                                uint32_t* flags, uint32_t* flags2);
 

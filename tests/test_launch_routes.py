@@ -49,3 +49,22 @@ for views, _ in {plans!r}:
 """)
     for (views, want), g in zip(plans, got):
         assert [tuple(v) for v in g] == want, views
+
+
+def test_cluster_paths():
+    """Small problems (cells x lights up to 2^22) on grids past 2048 columns or 128 a side: two brute-force
+    launches where the grid has few slices, else the column path; larger ones take the mark path."""
+    col2, col3 = ["k_col_count", "k_col_fill"], ["k_col_prep", "k_col_count", "k_col_fill"]
+    brute, mark = ["k_cluster_bf_count", "k_cluster_bf_fill"], ["k_cluster_geom", "k_cluster_mark"]
+    cases = [((16, 9, 24), 200, col2), ((16, 9, 24), 2000, col3), ((128, 16, 4), 600, col3),
+             ((256, 144, 1), 100, brute), ((80, 45, 1), 1000, brute), ((80, 45, 3), 300, brute),
+             ((80, 45, 1), 1200, mark), ((64, 36, 8), 200, col3), ((129, 8, 4), 600, col3),
+             ((255, 255, 2), 8, col3), ((200, 1, 1), 5000, col3), ((200, 1, 1), 300, col2),
+             ((64, 36, 24), 900, mark), ((80, 45, 24), 500, mark)]
+    got = routes(f"""
+for grid, n, _ in {cases!r}:
+    ds, cull = cull_pass(scene(n, 640, 360), grid)
+    result.append([k for k, _, _ in calls(lambda: cull.execute(ds))])
+""")
+    for (grid, n, want), g in zip(cases, got):
+        assert g[:len(want)] == want and (want == mark or len(g) == len(want)), (grid, n, g)
