@@ -621,11 +621,19 @@ HL_API hl_status hl_light_cull_clusters(hl_context* c, const GpuCameraUniforms* 
     if ((s = ensure(c, c->cull, sizeof(CullLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
     if ((s = ensure(c, c->hot, sizeof(HotLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
     if ((s = ensure(c, c->raw, cluster_raw_bytes((uint32_t)ncell))) != HL_OK) return s;
-    const ClusterPath path = cluster_path(p->grid_x, p->grid_y, p->grid_z, n);
+    ClusterPath path = cluster_path(p->grid_x, p->grid_y, p->grid_z, n);
     if (path == ClusterPath::kColumns) {
+        const std::string err = c->err;
         s = ensure(c, c->columns, column_scratch_bytes(p->grid_x, p->grid_y, p->grid_z, n));
-        if (s != HL_OK) return s;
-    } else if (path == ClusterPath::kMark) {
+        if (s == HL_ENOMEM) {  // the mark path's bitmask is smaller
+            (void)hipGetLastError();
+            c->err = err;
+            path = ClusterPath::kMark;
+        } else if (s != HL_OK) {
+            return s;
+        }
+    }
+    if (path == ClusterPath::kMark) {
         if ((s = ensure(c, c->geom, cluster_geom_bytes(ncol, (uint32_t)ncell))) != HL_OK) return s;
         if ((s = ensure(c, c->bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
         if ((s = ensure(c, c->summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;

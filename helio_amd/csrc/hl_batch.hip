@@ -227,7 +227,7 @@ hl_status build_plan(hl_plan* p) {
     }
     // The column path's blocks are shared out by cells x lights.  Its scratch
     // (12 bytes per block and light) is bounded over the plan: views past
-    // kBatchColScratch keep the mark path.
+    // kBatchColScratch, or that there is no memory for, keep the mark path.
     double work = 0.0;
     const auto view_work = [&](uint32_t v) {
         const hl_cluster_params& cp = p->cparams[v];
@@ -248,11 +248,18 @@ hl_status build_plan(hl_plan* p) {
         if ((s = plan_alloc(p, &b.cull, sizeof(CullLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
         const uint32_t aim = (uint32_t)(kBatchColBlocks * (view_work(v) / work)) + 1u;
         const BatchColumnPlan col = batch_column_plan(cp.grid_x, cp.grid_y, cp.grid_z, n, aim);
-        const bool columns = col.blocks != 0 && col_scratch + col.scratch <= kBatchColScratch;
+        bool columns = col.blocks != 0 && col_scratch + col.scratch <= kBatchColScratch;
         if (columns) {
-            if ((s = plan_alloc(p, &b.columns, col.scratch)) != HL_OK) return s;
-            col_scratch += col.scratch;
-        } else {
+            const std::string err = c->err;
+            columns = plan_alloc(p, &b.columns, col.scratch) == HL_OK;
+            if (columns) {
+                col_scratch += col.scratch;
+            } else {  // the mark path's bitmask is smaller
+                (void)hipGetLastError();
+                c->err = err;
+            }
+        }
+        if (!columns) {
             if ((s = plan_alloc(p, &b.geom, cluster_geom_bytes(ncol, ncell))) != HL_OK) return s;
             if ((s = plan_alloc(p, &b.bits, 4 * cluster_bits_words(ncell, n), true)) != HL_OK) return s;
             if ((s = plan_alloc(p, &b.summary, 4 * cluster_summary_words(ncell, n), true)) != HL_OK) return s;

@@ -1700,7 +1700,11 @@ static ColumnPlan column_plan(uint32_t ncol, uint32_t gz, uint32_t aim) {
 }
 // The scan reads 4 bytes per (block, light) and the candidates take 12 bytes
 // of scratch each in the worst case: the column path up to 2048 columns (128
-// a side) and 2^25 (block, light) pairs.
+// a side) and 2^25 (block, light) pairs, 403 MB (113 MB at 32x18x48 cells and
+// 16384 lights, where the mark path's bitmask takes 57).  That is a bound on
+// memory, not on speed: calls at it, us, columns / mark path, 64x32x24 cells and
+// 16384 lights 84 / 202, 64x32x48 101 / 285, 16x9x24 and 58000 145 / 208.  A
+// caller without the memory takes the mark path.
 static bool use_columns(uint32_t gx, uint32_t gy, uint32_t gz, uint64_t n) {
     const uint32_t ncol = gx * gy;
     return gx <= kColMaxSide && gy <= kColMaxSide && ncol <= kColMaxColumns &&

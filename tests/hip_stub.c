@@ -23,6 +23,7 @@ static struct {
 static int num_kernels;
 static char log_[kLog];
 static size_t log_len, alloc_limit = (size_t)-1, largest;
+static int last_error; /* of the last call that failed, until it is read */
 
 static void note(const char* what, const char* arg, uint32_t n) {
     int k = snprintf(log_ + log_len, kLog - log_len, "%s %s %u\n", what, arg, n);
@@ -83,7 +84,7 @@ int hipMalloc(void** p, size_t n) {
     if (n > alloc_limit) {
         *p = NULL;
         note("refused", "alloc", (uint32_t)(n >> 20));
-        return 2; /* hipErrorOutOfMemory */
+        return last_error = 2; /* hipErrorOutOfMemory */
     }
     uint8_t* q = mmap(NULL, n + kHead, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (q == MAP_FAILED) return 2;
@@ -140,7 +141,11 @@ int hipSetDevice(int d) {
     (void)d;
     return 0;
 }
-int hipGetLastError(void) { return 0; }
+int hipGetLastError(void) {
+    int e = last_error;
+    last_error = 0;
+    return e;
+}
 const char* hipGetErrorString(int e) {
     (void)e;
     return "stand-in";

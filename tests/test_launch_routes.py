@@ -68,3 +68,34 @@ for grid, n, _ in {cases!r}:
 """)
     for (grid, n, want), g in zip(cases, got):
         assert g[:len(want)] == want and (want == mark or len(g) == len(want)), (grid, n, g)
+
+
+def test_a_cull_without_memory_for_the_column_scratch_takes_the_mark_path():
+    """The column path reserves 12 bytes per (block, light), 398 MB for 45x45x24 cells and 16384 lights, the mark
+    path's bitmask takes 100: where the first allocation fails the call goes on with the second, and takes the
+    column path again when there is memory."""
+    single, plan = routes("""
+ds, cull = cull_pass(scene(16384, 640, 360), (45, 45, 24))
+row = []
+for limit in (200 << 20, NO_LIMIT):
+    row.append([k for k, _, _ in calls(lambda: cull.execute(ds), limit)])
+row.append(ctx.lib.raw["hl_last_error"](ctx.h).decode())
+result.append(row)
+sc = scene(16384, 640, 360)
+dv = upload_scene(ctx, sc)
+params = synth.cluster_params(ctx.lib, sc, grid=(45, 45, 24))
+view = BatchView(scene=dv, subset=ctx.upload(np.arange(16384, dtype=np.uint32)), num_lights=16384,
+                 out=ctx.alloc(640 * 360 * 16), clusters=params)
+row = []
+for limit in (200 << 20, NO_LIMIT):
+    stub.stub_reset(limit)
+    p = BatchPlan(ctx, dv.lights, 16384, [view])
+    row.append([k for k, _, _ in calls(p.launch)])
+    p.destroy()
+result.append(row)
+""")
+    assert single[0][:2] == ["k_cluster_geom", "k_cluster_mark"]
+    assert single[1] == ["k_col_prep", "k_col_count", "k_col_fill"]
+    assert single[2] == ""
+    assert plan[0][:2] == ["k_batch_geom", "k_batch_mark"]
+    assert plan[1][:3] == ["k_batch_col_prep", "k_batch_col_count", "k_batch_col_fill"]
