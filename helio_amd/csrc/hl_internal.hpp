@@ -250,12 +250,16 @@ __host__ __device__ inline bool fused_split(uint32_t num_blocks) { return num_bl
 // block tiles and lights: 256 36 / 40 / 44 (64 lights), 62 / 77 / 112 (512);
 // 1024 51 / 44 / 47, 82 / 83 / 111; 1350 61 / 53 / 54, 91 / 101 / 128; 2304
 // 79 / 57 / 55, 113 / 95 / 108; 3072 100 / 70 / 52, 156 / 124 / 116; 5120
-// 137 / 85 / 63, 201 / 140 / 138.  (The fused step keeps four up to its bound
-// above: its loss is returned in 64 bits, and other shares would move it by the
-// rounding of the radiance.)
+// 137 / 85 / 63, 201 / 140 / 138.  With thousands of lights two waves pay on
+// larger views too, with 2 / 1 in a crowded scene and in a sparse one: 3600
+// 53 / 39, 52 / 39 (64 lights), 174 / 225, 67 / 57 (1024), 295 / 412, 72 / 70
+// (2048), 1087 / 1546, 117 / 130 (8192); 5650 438 / 561, 93 / 74 (2048), 1670 /
+// 2267, 146 / 154 (8192); 8100 935 / 1147, 129 / 105 (4096).  (The fused step
+// keeps four up to its bound above: its loss is returned in 64 bits, and other
+// shares would move it by the rounding of the radiance.)
 __host__ __device__ inline uint32_t backward_share(uint32_t num_blocks, uint32_t num_lights) {
     if (num_blocks < 2048u && (num_blocks <= 512u || num_blocks <= 3ull * num_lights)) return 2u;
-    return num_blocks < 2560u ? 1u : 0u;
+    return num_blocks < 2560u || (num_blocks < 6144u && num_blocks <= 3ull * num_lights) ? 1u : 0u;
 }
 
 // The forward mode shares a wave tile's lights among the block's four waves, by

@@ -121,7 +121,7 @@ int hipGetSymbolAddress(void** p, const void* sym) {
 }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int block, size_t dyn) {
     (void)f, (void)block, (void)dyn;
-    *n = 4;
+    *n = 1 << 12; /* persistent launches: a block per item */
     return 0;
 }
 int hipDeviceGetAttribute(int* v, int attr, int dev) {
