@@ -225,7 +225,10 @@ hl_status build_plan(hl_plan* p) {
             if (st != HL_OK) return st;
         }
     }
-    // The column path's blocks are shared out by cells x lights.  Its scratch
+    // The column path's blocks are shared out by cells x lights, a block for
+    // every 512 lights of a view at the least while the views can all have that
+    // many (a 64^2 view of one column and 16384 lights beside a 1080p one: the
+    // count of its only block 105 us, the plan 164 -> 105).  Its scratch
     // (12 bytes per block and light) is bounded over the plan: views past
     // kBatchColScratch, or that there is no memory for, keep the mark path.
     double work = 0.0;
@@ -246,7 +249,8 @@ hl_status build_plan(hl_plan* p) {
         ViewBufs& b = p->bufs[v];
         if ((s = plan_alloc(p, &b.hot, sizeof(HotLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
         if ((s = plan_alloc(p, &b.cull, sizeof(CullLight) * (size_t)(n ? n : 1))) != HL_OK) return s;
-        const uint32_t aim = (uint32_t)(kBatchColBlocks * (view_work(v) / work)) + 1u;
+        const uint32_t aim = std::max((uint32_t)(kBatchColBlocks * (view_work(v) / work)) + 1u,
+                                      std::min(n / 512u, kBatchColBlocks / nv));
         const BatchColumnPlan col = batch_column_plan(cp.grid_x, cp.grid_y, cp.grid_z, n, aim);
         bool columns = col.blocks != 0 && col_scratch + col.scratch <= kBatchColScratch;
         if (columns) {

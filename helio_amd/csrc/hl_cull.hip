@@ -1085,6 +1085,11 @@ constexpr uint32_t kColMaxColumns = 2048;
 constexpr uint32_t kColBlocks = 512;
 constexpr uint32_t kColChunk = 16384;  // lights scanned at a time
 constexpr uint32_t kColThreads = 512;  // of a count block
+// of one where there are more blocks than fit the chip at once at 512 threads
+// (four per CU): what bounds them is then the rounds of blocks, and eight of half
+// the size fit
+constexpr uint32_t kColNarrow = 256;
+constexpr uint32_t kColResident = 1024;
 constexpr uint32_t kColInline = 512;   // lights every block bounds itself
 constexpr uint32_t kColInlineCells = 8192;
 constexpr uint32_t kColBatch = 512;    // candidates a fill block lists at a time
@@ -1210,13 +1215,13 @@ struct ColGeomSmem {
     ColCell cell[HL_MAX_SLICES];  // the block's cells
     SliceTab tab;
 };
-template <uint32_t CHUNK>
+template <uint32_t CHUNK, uint32_t NT>
 struct ColCountSmem {
     ColGeomSmem g;
     uint32_t words[CHUNK / 32];  // candidate bits of the chunk
     uint16_t list[CHUNK];        // the candidates, ascending, chunk-relative
-    uint32_t wave_sum[kColThreads / 64];
-    uint32_t cnt[kColThreads / 64][HL_MAX_SLICES];
+    uint32_t wave_sum[NT / 64];
+    uint32_t cnt[NT / 64][HL_MAX_SLICES];
 };
 struct ColFillSmem {
     uint32_t bits[HL_MAX_SLICES][kColBatch / 32];  // members of the batch per slice
@@ -1245,9 +1250,10 @@ __device__ __forceinline__ ColBlock col_block(const ClusterArgs& a, uint32_t blo
 // plane or a box per thread of the block's last two waves, which have no
 // lights to bound in the smallest problems) into LDS; the caller
 // synchronises.  Returns whether the column covers pixels (uniform).
+template <uint32_t NT>
 __device__ __forceinline__ bool col_setup(const ClusterArgs& a, const GpuCameraUniforms* __restrict__ cam,
                                           const ColBlock& c, ColGeomSmem& sm) {
-    const uint32_t t = threadIdx.x - (kColThreads - 64u);  // wraps: another wave
+    const uint32_t t = threadIdx.x - (NT - 64u);  // wraps: another wave
     if (t < c.nk) {
         ColumnGeom g;
         CellBox bx;
@@ -1262,7 +1268,7 @@ __device__ __forceinline__ bool col_setup(const ClusterArgs& a, const GpuCameraU
     }
     float l = 0.0f, r = 0.0f, b = 0.0f, tp = 0.0f;
     const bool on = column_rect(a, c.cx, c.cy, &l, &r, &b, &tp);
-    const uint32_t p = threadIdx.x - (kColThreads - 128u);
+    const uint32_t p = threadIdx.x - (NT - 128u);
     if (on && p < 4u) {
         // (l, b, l, t), (r, t, r, b), (l, t, r, t), (r, b, l, b)
         const float x0 = (p == 0u || p == 2u) ? l : r, y0 = (p == 0u || p == 3u) ? b : tp;
@@ -1418,10 +1424,11 @@ __global__ __launch_bounds__(64) void k_col_prep(ClusterArgs a, ColumnArgs p, ui
 // INLINE: the block bounds every light itself (a light per thread; the cone
 // terms come with the candidate's record), and the blocks share the shading
 // records.
-template <uint32_t CHUNK, bool INLINE>
+template <uint32_t CHUNK, uint32_t NT, bool INLINE>
 __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const ColumnArgs& p, uint32_t block,
-                                                uint32_t nblocks, ColCountSmem<CHUNK>& sm, uint32_t* inline_slices) {
-    constexpr uint32_t NT = kColThreads, kWaves = NT / 64u;
+                                                uint32_t nblocks, ColCountSmem<CHUNK, NT>& sm,
+                                                uint32_t* inline_slices) {
+    constexpr uint32_t kWaves = NT / 64u;
     static_assert(!INLINE || CHUNK == NT, "a light per thread");
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, n = a.num_lights;
     const ColBlock c = col_block(a, block, p.kb);
@@ -1436,7 +1443,7 @@ __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const Colu
         load_slices(a, sm.g.tab);
         __syncthreads();
     }
-    const bool on = col_setup(a, p.cam, c, sm.g);
+    const bool on = col_setup<NT>(a, p.cam, c, sm.g);
     const uint32_t key = column_key(c.cx >> p.shift, c.cy >> p.shift), k1 = c.k0 + c.nk - 1u;
     [[maybe_unused]] const bool part_column = c.nk != a.grid_z;
     if (INLINE && block == 0 && t == 0) {
@@ -1670,15 +1677,15 @@ __device__ __forceinline__ void col_fill_block(const ClusterArgs& a, const Colum
     }
 }
 
-template <uint32_t CHUNK, bool INLINE>
-__global__ __launch_bounds__(kColThreads) void k_col_count(ClusterArgs a, ColumnArgs p) {
-    __shared__ ColCountSmem<CHUNK> sm;
+template <uint32_t CHUNK, uint32_t NT, bool INLINE>
+__global__ __launch_bounds__(NT) void k_col_count(ClusterArgs a, ColumnArgs p) {
+    __shared__ ColCountSmem<CHUNK, NT> sm;
     uint32_t* is = nullptr;
     if constexpr (INLINE) {
         __shared__ uint32_t slices[CHUNK];
         is = slices;
     }
-    col_count_block<CHUNK, INLINE>(a, p, blockIdx.x, gridDim.x, sm, is);
+    col_count_block<CHUNK, NT, INLINE>(a, p, blockIdx.x, gridDim.x, sm, is);
 }
 
 template <bool SUMS>
@@ -1763,10 +1770,14 @@ size_t column_scratch_bytes(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t n) {
 // The column path of many views: the same three steps, a launch each, the
 // blocks of a view one after the other (base: first block of each view, and
 // the end).  The plan aims at a number of blocks for the whole batch, shared
-// out by cells x lights.  Lights are scanned kBatchColChunk at a time: the smaller list (8 KB against 32) lets four
-// blocks share a CU.  24 faces of 128^2 with 512 lights each and two 1032x1104
-// eyes with 4096: 7 + 23 + 8 us against the mark path's 51 (geometry 6, mark
-// 12, tail 11, count 9, fill 12).
+// out by cells x lights.  Lights are scanned kBatchColChunk at a time: the
+// smaller list (8 KB against 32) lets four blocks share a CU, or eight of half
+// the threads where the plan has more blocks than that (kColNarrow: a 4K frame
+// of 2040 columns and 16 lights 59.1 -> 54.1 us, four 1080p views of 2040 and 256
+// lights 145 -> 117; with 512 threads frames of many columns and few lights were
+// slower than on the mark path, 57.0 and 159).  24 faces of 128^2 with 512 lights
+// each and two 1032x1104 eyes with 4096: 7 + 23 + 8 us against the mark path's 51
+// (geometry 6, mark 12, tail 11, count 9, fill 12).
 struct BatchColumnView {
     ClusterArgs a;
     ColumnArgs p;
@@ -1794,12 +1805,13 @@ __global__ __launch_bounds__(64) void k_batch_col_prep(ConstColumnViews __restri
     col_prep_block(v.a, v.p, blockIdx.x - base[vi], v.nprep, v.nsum, tab);
 }
 
-__global__ __launch_bounds__(kColThreads) void k_batch_col_count(ConstColumnViews __restrict__ views,
-                                                                 const uint32_t* __restrict__ base, uint32_t nviews) {
-    __shared__ ColCountSmem<kBatchColChunk> sm;
+template <uint32_t NT>
+__global__ __launch_bounds__(NT) void k_batch_col_count(ConstColumnViews __restrict__ views,
+                                                        const uint32_t* __restrict__ base, uint32_t nviews) {
+    __shared__ ColCountSmem<kBatchColChunk, NT> sm;
     const uint32_t vi = view_of_block(base, nviews);
     const BatchColumnView& v = *(const BatchColumnView*)&views[vi];
-    col_count_block<kBatchColChunk, false>(v.a, v.p, blockIdx.x - base[vi], 0u, sm, nullptr);
+    col_count_block<kBatchColChunk, NT, false>(v.a, v.p, blockIdx.x - base[vi], 0u, sm, nullptr);
 }
 
 __global__ __launch_bounds__(256) void k_batch_col_fill(ConstColumnViews __restrict__ views,
@@ -1852,7 +1864,8 @@ hipError_t launch_batch_columns(hipStream_t s, const void* views, const uint32_t
     hipError_t e;
     k_batch_col_prep<<<prep_blocks, 64, 0, s>>>(v, prep_base, nviews);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    k_batch_col_count<<<col_blocks, kColThreads, 0, s>>>(v, col_base, nviews);
+    if (col_blocks > kColResident) k_batch_col_count<kColNarrow><<<col_blocks, kColNarrow, 0, s>>>(v, col_base, nviews);
+    else k_batch_col_count<kColThreads><<<col_blocks, kColThreads, 0, s>>>(v, col_base, nviews);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     k_batch_col_fill<<<col_blocks, 256, 0, s>>>(v, col_base, nviews);
     return hipGetLastError();
@@ -2455,7 +2468,7 @@ hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCam
         (void)column_scratch((uint8_t*)w.columns, ncol, a.grid_z, a.num_lights, cp.blocks, &p);
         hipError_t e;
         if (column_inline(ncell, a.num_lights)) {
-            k_col_count<kColInline, true><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+            k_col_count<kColInline, kColThreads, true><<<cp.blocks, kColThreads, 0, s>>>(a, p);
             if ((e = hipGetLastError()) != hipSuccess) return e;
             k_col_fill<false><<<cp.blocks, 256, 0, s>>>(a, p);
             return hipGetLastError();
@@ -2464,9 +2477,9 @@ hipError_t launch_cluster_cull(hipStream_t s, const ClusterArgs& a, const GpuCam
             a, p, column_groups(ncol) * a.grid_z);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (ncol <= kColMaxColumns)
-            k_col_count<kColChunk, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
-        else  // many small blocks: the smaller list lets four share a CU
-            k_col_count<kBatchColChunk, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+            k_col_count<kColChunk, kColThreads, false><<<cp.blocks, kColThreads, 0, s>>>(a, p);
+        else  // many blocks with few lights
+            k_col_count<kBatchColChunk, kColNarrow, false><<<cp.blocks, kColNarrow, 0, s>>>(a, p);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         k_col_fill<true><<<cp.blocks, 256, 0, s>>>(a, p);
         return hipGetLastError();

@@ -123,3 +123,28 @@ for w, h, n, _ in {cases!r}:
 """)
     for c, g in zip(cases, got):
         assert g == [c[3]], c
+
+
+def test_batched_column_blocks():
+    """More column blocks than the chip holds at 512 threads are launched at 256; a view of few columns and many
+    lights has a block per 512 lights while every view can."""
+    few, many, deep, deeps = routes("""
+def view(n, w, h, grid):
+    sc = scene(n, w, h)
+    ds = upload_scene(ctx, sc)
+    return BatchView(scene=ds, subset=ctx.upload(np.arange(n, dtype=np.uint32)), num_lights=n,
+                     out=ctx.alloc(w * h * 16), clusters=synth.cluster_params(ctx.lib, sc, grid=grid))
+
+for views in ([(64, 640, 360, (10, 6, 24))] * 2, [(64, 640, 360, (10, 6, 24))] * 18,
+              [(16384, 640, 360, (30, 17, 24)), (16384, 64, 64, (1, 1, 24))],
+              [(16384, 640, 360, (30, 17, 24))] + [(16384, 64, 64, (1, 1, 24))] * 63):
+    made = {v: view(*v) for v in views}
+    pool = max(made.values(), key=lambda v: v.num_lights)
+    plan = BatchPlan(ctx, pool.scene.lights, pool.num_lights, [made[v] for v in views])
+    result.append([(v, b) for k, v, b in calls(plan.launch) if k == "k_batch_col_count"])
+    plan.destroy()
+""")
+    assert [v for v, _ in few] == [[512]] and [v for v, _ in many] == [[256]]
+    assert many[0][1] == 18 * 60
+    assert deep[0][1] == 2 * 510 + 24  # 511 aimed at and 32, a block per slice
+    assert deeps[0][1] == 510 + 63 * 8
