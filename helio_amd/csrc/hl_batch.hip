@@ -50,7 +50,8 @@ struct ViewBufs {
 // Blocks the column path's views share, and its scratch over a plan.
 // 512 blocks are aimed at: whole columns on all but the smallest grids, where
 // a few blocks per view are enough (256 and 1024 measured the same for a frame
-// of 24 faces and two eyes: 24.1 and 25.8 us counting, against 24.2).  1 GiB holds the scratch of the 50-view frame of 48 faces and two
+// of 24 faces and two eyes: 24.1 and 25.8 us counting, against 24.2).  1 GiB
+// holds the scratch of the 50-view frame of 48 faces and two
 // 2064x2208 eyes four times over.
 constexpr uint32_t kBatchColBlocks = 512;
 constexpr size_t kBatchColScratch = 1ull << 30;
@@ -320,7 +321,10 @@ hl_status build_plan(hl_plan* p) {
     if ((s = plan_alloc(p, &p->d_cols, batch_column_view_size() * p->col_views.size())) != HL_OK) return s;
     if ((s = plan_alloc(p, &p->d_markq, mark_queue_bytes(p->total_lights))) != HL_OK) return s;
     const std::pair<uint32_t**, const std::vector<uint32_t>*> bases[] = {
-        {&p->d_light_base, &light_base}, {&p->d_cell_base, &cell_base}, {&p->d_prep_base, &prep_base}, {&p->d_col_base, &col_base}};
+        {&p->d_light_base, &light_base},
+        {&p->d_cell_base, &cell_base},
+        {&p->d_prep_base, &prep_base},
+        {&p->d_col_base, &col_base}};
     for (const auto& b : bases) {
         if ((s = plan_alloc(p, (void**)b.first, 4 * b.second->size())) != HL_OK) return s;
         HL_HIP(c, hipMemcpy(*b.first, b.second->data(), 4 * b.second->size(), hipMemcpyHostToDevice));

@@ -1521,7 +1521,8 @@ __device__ __forceinline__ void col_count_block(const ClusterArgs& a, const Colu
         p.raw[c.col + c.ncol * (c.k0 + t)] = v;
         const uint32_t capped = (a.cap && v > a.cap) ? a.cap : v;
         if (!INLINE && capped)
-            atomicAdd(p.gsum + (size_t)(c.k0 + t) * ((c.ncol + kColGroup - 1u) / kColGroup) + c.col / kColGroup, capped);
+            atomicAdd(p.gsum + (size_t)(c.k0 + t) * ((c.ncol + kColGroup - 1u) / kColGroup) + c.col / kColGroup,
+                      capped);
     }
     if (t == 0u) p.num_cand[block] = done;
     // the shading records, last: no wait stands on them

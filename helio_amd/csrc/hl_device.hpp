@@ -601,8 +601,8 @@ __device__ __forceinline__ float dpp_sum4(float v0, float v1, float v2, float v3
     return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
-// min and max of three coordinates over the lanes with `take` set (+inf / -inf
-// when none; no NaN).  The six keys (a maximum as the minimum of complements)
+// min and max of three coordinates over the lanes with `take` set: at least one
+// lane, or the results are NaN (the identity key's); no NaN among them.  The six keys (a maximum as the minimum of complements)
 // halve with the lanes in the first three steps, as in dpp_sum4: lane bit 0
 // picks minimum or maximum, bit 1 x or y, bit 2 those or z: 13 VALU
 // instructions fewer than six reductions.  Integer keys with their identity as

@@ -291,8 +291,8 @@ __host__ __device__ inline bool forward_split(uint32_t grid_mode, uint32_t width
 // Work items of a single-view shading launch of MODE (a ShadeMode with its
 // flags): the shared forward and the fused mode when split share each wave
 // tile's lights among a block's four waves, so their items are wave tiles (four
-// per block tile), and the backward mode likewise by its share.  A batched launch shares under the fused
-// mode only.
+// per block tile), and the backward mode likewise by its share.  A batched
+// launch shares under the fused mode only.
 template <int MODE>
 __host__ __device__ inline uint32_t shade_items(const ShadeArgs& a) {
     constexpr int M = MODE & kModeMask;

@@ -269,8 +269,10 @@ struct LightShare {
 };
 // Waves that share a tile by the ordinals of its visited lights: f is called,
 // and with kept a record stored, only where ord % (mask + 1) == value.  The
-// lights of the other waves cost a bit of the ballot here, no staging and no
-// turn of the loop (512^2 fused step 85 -> 80 us a call, 773x431 backward 91 -> 87).
+// lights of the other waves cost a bit of the ballot here and no turn of the
+// loop, and with kept no staging (without, a light is staged as it is loaded,
+// ahead of the ballot).  512^2 fused step 85 -> 80 us a call, 773x431 backward
+// 91 -> 87.
 struct OrdinalShare {
     uint32_t mask, value;
     uint32_t ord = 0u;  // lights visited so far
