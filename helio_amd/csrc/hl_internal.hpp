@@ -266,30 +266,33 @@ __host__ __device__ inline uint32_t backward_share(uint32_t num_blocks, uint32_t
 // the light's index modulo 4, where a wave that walks its list alone is one
 // long serial chain and the view has too few wave tiles to hide it; the price is
 // the tile's set-up and walk, four times.  Worth it by the lights of a tile,
-// which the host does not know: by a light for every 512 pixels (448 past 2^18),
-// up to 15 * 2^16 pixels, on tile lists, which end at 64 lights, up to 2^17.
-// Shading calls, us, unshared / shared, in a crowded scene, and frames (cull and
-// shading) in a sparse one: clusters 128^2 8.9 / 7.8, 27.4 / 23.0 (64 lights),
-// 33 / 16, 68 / 41 (1024); 256^2 8.5 / 9.4 (64), 9.7 / 9.5, 31 / 26 (128); 512^2
-// 16.6 / 21.9 (256), 25.9 / 23.4, 89 / 55 (512); 960^2 79 / 77 (1024), 107 / 89
-// (2048), 174 / 125 (4096); 1024^2 64 / 75, 78 / 96 (2048), 287 / 186, 81 / 117
-// (16384).  Over eight sizes from 640x480 to 1300x731 with 1024 to 4096 lights and
-// five scenes the rule's calls are up to 1.8 times as fast, three of 185 slower (by
-// 5 % at most); with 8192 and 16384, in scenes wide for them, 0.58 to 2.3 times as
-// fast, 1.13 in the mean.  Tiles 256^2 7.3 / 7.3 (64), 10.6 / 8.6,
-// 30 / 20 (256); 352^2 10.7 / 12.5 (256), 18.8 / 14.3, 25.3 / 28.2 (1024); 512^2
-// 11.1 / 16.1 (256), 19.2 / 18.3, 29.4 / 34.4 (1024).  (By a light for 1400 pixels
-// alone, up to 2^20, a 1024^2 view of 749 lights took 56 us for 29, on tiles 48
-// for 23.)  The shadowed and extended modes, whose light costs several times as
-// much, were not tried.
+// which the host does not know; the line lies where scenes of several densities
+// break even together.  Clusters: a light for every 1024 pixels up to 2^18, where
+// the block tiles are one round of the 1280 resident blocks, for every 448 up to
+// 15 * 2^16; tile lists, which end at 64 lights, every 512 up to 2^17.  Unshared /
+// shared, us, a shading call in a sparse scene, then frames (cull and shading) in
+// two crowded ones.  Clusters: 128^2 7.7 / 7.5, 21 / 20, 23 / 22 (16 lights), 33 / 16,
+// 68 / 41, 52 / 38 (1024); 256^2 7.2 / 8.9, 20 / 21, 22 / 22 (16), 8.5 / 9.4, 26 / 23,
+// 31 / 27 (64); 512^2 12.2 / 19.5, 37 / 38, 43 / 39 (128), 16.6 / 21.9, 55 / 44, 61 / 44
+// (256), the 256-light fp32 one 44 / 36 shading; 960^2 79 / 77 (1024), 107 / 89 (2048),
+// 174 / 125 (4096); 1024^2 64 / 75, 78 / 96 (2048), 287 / 186, 81 / 117 (16384).  Over
+// eight sizes from 640x480 to 1300x731 with 1024 to 4096 lights and five scenes the
+// rule's calls are up to 1.8 times as fast, three of 185 slower (by 5 % at most); with
+// 8192 and 16384, in scenes wide for them, 0.58 to 2.3 times as fast, 1.13 in the
+// mean.  Tiles: 256^2 7.3 / 7.3, 18.5 / 15.7, 17.9 / 16.0 (64); 352^2 8.8 / 11.4, 25 / 21,
+// 20 / 21 (128), 10.7 / 12.5, 30 / 24, 24 / 23 (256); 512^2 11.1 / 16.1, 32 / 29, 25 / 28
+// (256).  (A light for every 1400 pixels up to 2^20, on either grid: a 1024^2 view of
+// 749 lights 56 us for 29, on tiles 48 for 23.)  The shadowed and extended modes,
+// whose light costs several times as much, were not tried.
 // The rule and the shares depend on the view's size, its lights and the kind of
 // grid only, so every path shading a view (single, batched, any tile shape) adds
 // the same sums.
 __host__ __device__ inline bool forward_split(uint32_t grid_mode, uint32_t width, uint32_t height,
                                               uint32_t num_lights) {
     const uint64_t px = (uint64_t)width * height;
-    if (num_lights < 16u || px > (grid_mode == HL_GRID_TILES ? 1u << 17 : 15u << 16)) return false;
-    return px <= (px <= (1u << 18) ? 512ull : 448ull) * num_lights;
+    if (num_lights < 16u) return false;
+    if (grid_mode == HL_GRID_TILES) return px <= (1u << 17) && px <= 512ull * num_lights;
+    return px <= (15u << 16) && px <= (px <= (1u << 18) ? 1024ull : 448ull) * num_lights;
 }
 
 // Work items of a single-view shading launch of MODE (a ShadeMode with its

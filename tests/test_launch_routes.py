@@ -11,11 +11,11 @@ def test_forward_shares_wave_tiles_only_where_that_is_faster():
     two forms took the same time, on clusters and on tile lists (which end at 64 lights)."""
     cases = [  # width, height, lights, shared on clusters, on tiles
         (64, 64, 4, False, False), (32, 32, 15, False, False), (64, 64, 16, True, True),
-        (128, 128, 31, False, False), (128, 128, 64, True, True), (256, 256, 64, False, False),
-        (256, 256, 128, True, True), (333, 177, 16, False, False), (352, 352, 512, True, True),
-        (512, 512, 256, False, False), (512, 512, 512, True, False), (720, 720, 1024, False, False),
-        (720, 720, 4096, True, False), (1300, 731, 2048, False, False), (1300, 731, 2554, True, False),
-        (1024, 1024, 749, False, False), (1024, 1024, 16384, False, False),
+        (128, 128, 31, True, False), (128, 128, 64, True, True), (256, 256, 16, False, False),
+        (256, 256, 64, True, False), (256, 256, 128, True, True), (333, 177, 16, False, False),
+        (352, 352, 512, True, True), (512, 512, 128, False, False), (512, 512, 256, True, False),
+        (720, 720, 1024, False, False), (720, 720, 4096, True, False), (1300, 731, 2048, False, False),
+        (1300, 731, 2554, True, False), (1024, 1024, 749, False, False), (1024, 1024, 16384, False, False),
     ]
     got = routes(f"""
 for w, h, n, _, _ in {cases!r}:
